@@ -112,9 +112,10 @@ int32_t tensor_gguf_packed_v1(const TensorCallV1 *call, TensorErrorV1 *error);
  * (a decoder's gate and up projections, or q, k and v).  No counterpart in the
  * reference: there every linear is its own gemv_packed launch
  * (benchmarks/kernels/showcase/kernels.py:114-119).  The group is one launch
- * of the Q4_K M = 1 kernel when K is a multiple of 4096; for other encodings
- * and shapes it is c launches of tensor_gguf_gemv_v1's kernels in order on the
- * stream.  Arguments, in order:
+ * of the Q4_K / Q5_K M = 1 kernel when K is a multiple of 4096 (at most 16384), else one
+ * launch of the matrix-core decode kernel; a single matrix, and groups at M = 1 of 2^25
+ * elements or more whose K is a multiple of 2048, are c launches of tensor_gguf_gemv_v1's
+ * kernels in order on the stream.  Arguments, in order:
  *   0        x     buffer fp16  [M, K], 1 <= M <= TENSOR_GGUF_GEMV_MAX_M
  *   2i+1     w_i   buffer uint8 [N_i, K/QK*BLOCK]
  *   2i+2     out_i buffer [M, N_i], one dtype (fp16 or fp32) for all i
@@ -240,7 +241,8 @@ int32_t tensor_gguf_gemv_variant_v1(const TensorCallV1 *call, TensorErrorV1 *err
  * (src/tensor/compiler/webgpu/schedules/packed_integer.py:26-31, epilogue
  * :204-205); the showcase path would take two gemv_packed launches and an
  * elementwise kernel.  One launch: the Q4_K M = 1 kernel with gate and up rows
- * in one workgroup when K is a multiple of 4096 (at most 16384), else the
+ * (and Q5_K) in one workgroup when K is a multiple of 4096 (at most 16384), else the matrix-core
+ * decode kernel with gate and up tiles in turn; small matrices take the
  * generic decode kernels with a gate / up row pair per wave.  Arguments:
  *   0 x      buffer fp16  [M, K], 1 <= M <= TENSOR_GGUF_GEMV_MAX_M
  *   1 w_gate buffer uint8 [N, K/QK*BLOCK]

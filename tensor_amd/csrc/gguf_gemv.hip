@@ -1010,6 +1010,7 @@ static hipError_t launch_swiglu_out(const GemvArgs& a, const uint8_t* w_up, hipS
 }
 
 hipError_t launch_gemv_swiglu(const GemvArgs& a, const void* w_up, hipStream_t stream) {
+  if (gemv_rows_pair(a)) return launch_gemv_rows(&a, 1, w_up, stream);
   if (a.type == kQ4_K || a.type == kQ5_K) {
     bool handled = false;
     const hipError_t status = launch_gemv_q4k_swiglu_fast(a, w_up, stream, &handled);
@@ -1020,6 +1021,7 @@ hipError_t launch_gemv_swiglu(const GemvArgs& a, const void* w_up, hipStream_t s
 }
 
 hipError_t launch_gemv(const GemvArgs& a, hipStream_t stream) {
+  if (gemv_rows_single(a)) return launch_gemv_rows(&a, 1, nullptr, stream);
   if (a.type == kQ4_K || a.type == kQ5_K || a.type == kQ6_K) {
     bool handled = false;
     const hipError_t status = a.type == kQ4_K   ? launch_gemv_q4k_fast(a, stream, &handled)

@@ -485,23 +485,14 @@ __device__ __forceinline__ int sum_slot(int run) { return (run & ~3) | ((run & 1
 
 __device__ __forceinline__ uint32_t half2_bits(half2_t v) { return __builtin_bit_cast(uint32_t, v); }
 
-// PAIR = 1 (SwiGLU) or 2 (two outputs): the workgroup's two tile slots are tile blockIdx.x of w
-// and the same tile of w2, a second matrix of the same shape. PAIR = 1: the wave that sums the w
-// (gate) tile also sums the w2 (up) tile's partials and stores silu(gate) * up to out. PAIR = 2:
-// each tile is stored, to out and out2 (the grouped GEMV of two equal matrices in one launch).
-//
 // SPLITS > 1 (x of the whole row does not fit in LDS): K is cut into SPLITS equal ranges, and
 // workgroup SPLITS g + s takes range s of tile group g, staging only that range of x.  Its
 // reduced tiles are fp32 partial sums, stored to part[s][m][n]; gemv_q4k_sec_reduce adds the
 // ranges in order.
-template <int M, typename OutT, int PAIR = 0, bool XFIRST = true, int SPLITS = 1>
+template <int M, typename OutT, bool XFIRST = true, int SPLITS = 1>
 __global__ __launch_bounds__(1024) void gemv_q4k_sec(const _Float16* __restrict__ x, const uint8_t* __restrict__ w,
                                                      OutT* __restrict__ out, int n_rows, int k, int tiles,
-                                                     const uint8_t* __restrict__ w2 = nullptr,
-                                                     OutT* __restrict__ out2 = nullptr,
                                                      float* __restrict__ part = nullptr) {
-  constexpr bool SWIGLU = PAIR == 1;
-  static_assert(SPLITS == 1 || PAIR == 0, "K ranges split across workgroups store one matrix's partials");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   constexpr int XCH = 8;  // x chunks per thread (the host checks M * K / 8 <= XCH * threads)
   const int row_bytes = (k >> 8) * 144;  // the whole row
@@ -536,8 +527,8 @@ __global__ __launch_bounds__(1024) void gemv_q4k_sec(const _Float16* __restrict_
       }
     }
   }
-  const int tile = PAIR ? group : group * tiles + t;
-  const uint8_t* base = (PAIR && t == 1 ? w2 : w) + (size_t)min(tile * 16 + n, n_rows - 1) * row_bytes +
+  const int tile = group * tiles + t;
+  const uint8_t* base = w + (size_t)min(tile * 16 + n, n_rows - 1) * row_bytes +
                         (split * KW + q) * 576 + 16 * g;
   uint4 v[9];
   auto load_weights = [&]() {
@@ -656,17 +647,10 @@ __global__ __launch_bounds__(1024) void gemv_q4k_sec(const _Float16* __restrict_
   float4v_t* partial = reinterpret_cast<float4v_t*>(lds);
   partial[wv * 64 + lane] = total;
   __syncthreads();
-  if (q != 0 || tile * 16 >= n_rows || (SWIGLU && t != 0)) return;
+  if (q != 0 || tile * 16 >= n_rows) return;
   // wave (t, 0) sums its tile's K ranges in order and stores it
   float4v_t sum = partial[t * KW * 64 + lane];
   for (int p = 1; p < KW; ++p) sum += partial[(t * KW + p) * 64 + lane];
-  if constexpr (SWIGLU) {
-    float4v_t up = partial[KW * 64 + lane];
-    for (int p = 1; p < KW; ++p) up += partial[(KW + p) * 64 + lane];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sum[i] = swiglu(sum[i], up[i]);
-  }
-  OutT* dst = PAIR == 2 && t == 1 ? out2 : out;
   const int col = tile * 16 + n;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -675,7 +659,7 @@ __global__ __launch_bounds__(1024) void gemv_q4k_sec(const _Float16* __restrict_
       if constexpr (SPLITS > 1)
         part[((size_t)split * M + m) * n_rows + col] = sum[i];
       else
-        store_out<OutT>(dst, (size_t)m * n_rows + col, sum[i]);
+        store_out<OutT>(out, (size_t)m * n_rows + col, sum[i]);
     }
   }
 }
@@ -939,11 +923,11 @@ static hipError_t launch_sec(const GemvArgs& a, hipStream_t stream, int per, boo
   const size_t lds = sec_lds_bytes(M, a.k, per * kw);
   const int grid = (tiles + per - 1) / per;
   if (xfirst)
-    hipLaunchKernelGGL((gemv_q4k_sec<M, OutT, 0, true>), dim3(grid), dim3(threads), lds, stream,
+    hipLaunchKernelGGL((gemv_q4k_sec<M, OutT, true>), dim3(grid), dim3(threads), lds, stream,
                        static_cast<const _Float16*>(a.x), static_cast<const uint8_t*>(a.w), static_cast<OutT*>(a.out),
                        a.n, a.k, per);
   else
-    hipLaunchKernelGGL((gemv_q4k_sec<M, OutT, 0, false>), dim3(grid), dim3(threads), lds, stream,
+    hipLaunchKernelGGL((gemv_q4k_sec<M, OutT, false>), dim3(grid), dim3(threads), lds, stream,
                        static_cast<const _Float16*>(a.x), static_cast<const uint8_t*>(a.w), static_cast<OutT*>(a.out),
                        a.n, a.k, per);
   return hipGetLastError();
@@ -959,9 +943,9 @@ static hipError_t launch_sec_split_cfg(const GemvArgs& a, hipStream_t stream, in
   const size_t lds = sec_lds_bytes(M, ks, per * kw);
   const int groups = (tiles + per - 1) / per;
   float* part = static_cast<float*>(a.workspace);
-  hipLaunchKernelGGL((gemv_q4k_sec<M, OutT, 0, true, SPLITS>), dim3(groups * SPLITS), dim3(threads), lds, stream,
+  hipLaunchKernelGGL((gemv_q4k_sec<M, OutT, true, SPLITS>), dim3(groups * SPLITS), dim3(threads), lds, stream,
                      static_cast<const _Float16*>(a.x), static_cast<const uint8_t*>(a.w), static_cast<OutT*>(a.out),
-                     a.n, a.k, per, nullptr, nullptr, part);
+                     a.n, a.k, per, part);
   hipError_t status = hipGetLastError();
   if (status != hipSuccess) return status;
   hipLaunchKernelGGL((gemv_q4k_sec_reduce<SPLITS, OutT>), dim3((a.n + 255) / 256, M), dim3(256), 0, stream, part,
@@ -977,37 +961,6 @@ static hipError_t launch_sec_split(const GemvArgs& a, hipStream_t stream, int pe
     if (!a.workspace || a.workspace_bytes < sec_split_bytes(a, splits)) return hipErrorInvalidValue;
     return splits == 2 ? launch_sec_split_cfg<M, 2, OutT>(a, stream, per)
                        : launch_sec_split_cfg<M, 4, OutT>(a, stream, per);
-  }
-}
-
-// SwiGLU pairs at 2 <= M <= 8 on the sector-aligned kernel: one gate tile and the same up tile
-// per workgroup (2 x K/1024 waves, so K <= 8192), x in LDS.
-template <int M, typename OutT, int PAIR>
-static hipError_t launch_sec_pair(const GemvArgs& a, const void* w2, void* out2, hipStream_t stream, bool* handled) {
-  *handled = false;
-  const int kw = a.k / 1024, tiles = (a.n + 15) / 16, threads = 2 * kw * 64;
-  if (a.k % 1024 != 0 || kw > 8) return hipSuccess;
-  const size_t lds = sec_lds_bytes(M, a.k, 2 * kw);
-  if ((long)M * a.k / 8 > 8L * threads || lds > kSecMaxLds) return hipSuccess;
-  *handled = true;
-  hipLaunchKernelGGL((gemv_q4k_sec<M, OutT, PAIR, false>), dim3(tiles), dim3(threads), lds, stream,
-                     static_cast<const _Float16*>(a.x), static_cast<const uint8_t*>(a.w), static_cast<OutT*>(a.out),
-                     a.n, a.k, 2, static_cast<const uint8_t*>(w2), static_cast<OutT*>(out2));
-  return hipGetLastError();
-}
-
-template <typename OutT, int PAIR>
-static hipError_t launch_pair_multirow(const GemvArgs& a, const void* w2, void* out2, hipStream_t stream,
-                                       bool* handled) {
-  switch (a.m) {
-    case 2: return launch_sec_pair<2, OutT, PAIR>(a, w2, out2, stream, handled);
-    case 3: return launch_sec_pair<3, OutT, PAIR>(a, w2, out2, stream, handled);
-    case 4: return launch_sec_pair<4, OutT, PAIR>(a, w2, out2, stream, handled);
-    case 5: return launch_sec_pair<5, OutT, PAIR>(a, w2, out2, stream, handled);
-    case 6: return launch_sec_pair<6, OutT, PAIR>(a, w2, out2, stream, handled);
-    case 7: return launch_sec_pair<7, OutT, PAIR>(a, w2, out2, stream, handled);
-    case 8: return launch_sec_pair<8, OutT, PAIR>(a, w2, out2, stream, handled);
-    default: *handled = false; return hipSuccess;
   }
 }
 
@@ -1163,18 +1116,6 @@ bool gemv_q4k_group_supported(int m, int k, int n) {
   return m == 1 && k % 4096 == 0 && k <= 4 * 4096 && (uint64_t)n * (uint64_t)(k / 256) * 176u < (1ull << 32);
 }
 
-// Up to M = 4 (gate + up 2 x 12288 x 4096 at M = 4: 17.4 us against 21.4 us for two launches; at
-// M = 8 the 64 KB of x staged for two tiles per workgroup makes the pair slower, 24.6 against 23.1).
-bool gemv_q4k_pair_supported(const GemvArgs* a, int count) {
-  return count == 2 && a[0].type == kQ4_K && a[0].m >= 2 && a[0].m <= 4 && a[1].n == a[0].n &&
-         a[0].k % 1024 == 0 && a[0].k <= 8192;
-}
-
-hipError_t launch_gemv_q4k_pair(const GemvArgs* a, hipStream_t stream, bool* handled) {
-  return a[0].out_half ? launch_pair_multirow<_Float16, 2>(a[0], a[1].w, a[1].out, stream, handled)
-                       : launch_pair_multirow<float, 2>(a[0], a[1].w, a[1].out, stream, handled);
-}
-
 hipError_t launch_gemv_q4k_group(const GemvArgs* a, int count, hipStream_t stream, int waves) {
   if (a[0].type == kQ5_K)
     return a[0].out_half ? launch_m1_group<_Float16, kQ5_K>(a, count, stream, waves)
@@ -1206,9 +1147,6 @@ static hipError_t launch_m1_swiglu_waves(const GemvArgs& a, const void* w_up, hi
 
 hipError_t launch_gemv_q4k_swiglu_fast(const GemvArgs& a, const void* w_up, hipStream_t stream, bool* handled,
                                        int waves) {
-  if (a.type == kQ4_K && a.m >= 2)
-    return a.out_half ? launch_pair_multirow<_Float16, 1>(a, w_up, nullptr, stream, handled)
-                      : launch_pair_multirow<float, 1>(a, w_up, nullptr, stream, handled);
   *handled = gemv_q4k_group_supported(a.m, a.k, a.n);
   if (!*handled) return hipSuccess;
   if (a.type == kQ5_K)

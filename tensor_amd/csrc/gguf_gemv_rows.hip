@@ -1,0 +1,634 @@
+// Decode GEMV on matrix cores, every encoding, any K the encoding allows, 1 <= M <= 8 rows of
+// fp16 activations: out[m, n] = sum_k x[m, k] * W[n, k], up to three matrices that share x in
+// one launch, or a gate / up pair with the SwiGLU epilogue.
+//
+// Each lane owns whole pieces of one weight row (a unit of 64 or 128 elements: two 32-element
+// blocks, or a quarter or half super-block), so that a piece's scale is a value of the lane's
+// own and is applied once per 16 or 32 elements in fp32.  v_mfma_f32_16x16x32_f16 does the
+// products all the same: its B operand takes 8 codes from every lane (lane n + 16 g: row n of a
+// 16-row tile, piece g of four that follow each other), and its A operand holds the activations
+// block-diagonally, row 4 g + m being x[m] over piece g and zero over the other three.  Result
+// rows 4 g .. 4 g + 3 are then the four activation rows' sums over piece g alone, and they lie in
+// just the lanes that own piece g.  Three quarters of the multiplies are by zero, which a decode
+// GEMV can afford: at M <= 4 a SIMD spends 16 of its cycles per 512 weights on them, against the
+// ~60 of the decode (M > 4 takes a second MFMA for rows 4..7), while a vector dot product
+// would spend M / 2 instructions per weight pair and read M activations per weight from LDS.
+//
+// Codes enter the MFMA as fp16 subnormals (code * 2^-24: v_perm_b32 widens bytes with a zero
+// high byte; the MFMA keeps subnormals), so nothing is biased and cancelled; encodings with a
+// constant offset subtract it exactly (v_pk_add_f16).  Minimums multiply the sums of x over their
+// 16 or 32 elements, which come from an MFMA of the same activations with ones.
+//
+// A workgroup owns one or a few 16-row tiles and splits K over its waves; a wave fetches 16 rows x 256
+// columns at a time in 16-byte pieces along the rows (lane-owned pieces read straight from memory
+// touch a cache line per lane and stop at 2 TB/s), passes them to their owning lanes through an LDS
+// area of its own, and requests the next ones before it multiplies.  The activations are staged
+// in LDS in slices (all of K where it fits), padded with zeros to whole steps; the first are requested
+// ahead of the first weights and waited for behind them.  Partial sums meet in LDS in range order.
+//
+// What bounds it: the stream at large shapes (Q8_0 12288 x 4096 at M = 4: 13.1 us, 4.1 TB/s;
+// 22.9 on the vector kernel), below ~8 MB the chain from launch to store (x, weights, LDS, MFMAs,
+// partial sums; ~2.5 us over an empty launch).  Instructions count there: integer divisions, branchy
+// bounds checks and unrolled variants of this kernel that ran each instruction once cost up to 3 us
+// in fetching them.  Microseconds per launch (graph replays, weights rotated), vector kernels ->
+// here: Q6_K 4096 x 12288 22.3 -> 13.5 (M = 4), 64.0 -> 17.9 (M = 8); Q4_0 12288 x 4096 55.2 -> 11.3
+// (M = 8); Q5_0 6912 x 2560 10.2 -> 6.8 (M = 2); Q3_K 2560 x 6912 10.4 -> 7.4 (M = 1); Q5_K SwiGLU
+// pair 2 x 6912 x 2560 33.4 -> 9.0 (M = 1), 90.6 -> 11.3 (M = 8).  Measured and not kept: two
+// row tiles per wave (spills), shares of the steps that cross tiles (code size), lanes
+// without activations masked off instead of reading zeros (1-3% slower).
+#include <algorithm>
+
+#include "gguf_common.h"
+#include "gguf_launch.h"
+
+namespace tensor_gguf {
+namespace {
+
+typedef float float4v __attribute__((ext_vector_type(4)));
+
+// Bytes 0 and 1 of c as the fp16 subnormal pair (c0, c1) * 2^-24; bytes 2 and 3 likewise.
+__device__ __forceinline__ uint32_t sub01(uint32_t c) { return __builtin_amdgcn_perm(0u, c, 0x0C010C00u); }
+__device__ __forceinline__ uint32_t sub23(uint32_t c) { return __builtin_amdgcn_perm(0u, c, 0x0C030C02u); }
+
+// The eight byte codes of two dwords as an MFMA operand, OFFSET (< 1024) subtracted from each.
+template <int OFFSET>
+__device__ __forceinline__ half8_t operand(uint32_t lo, uint32_t hi) {
+  uint32_t v[4] = {sub01(lo), sub23(lo), sub01(hi), sub23(hi)};
+  if constexpr (OFFSET != 0) {
+    constexpr uint32_t off = 0x80008000u | (uint32_t)OFFSET | ((uint32_t)OFFSET << 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __builtin_bit_cast(uint32_t, as_half2(v[i]) + as_half2(off));
+  }
+  return __builtin_bit_cast(half8_t, make_uint4(v[0], v[1], v[2], v[3]));
+}
+
+// Bit i (0..3) of v to bit 4 of byte i.
+__device__ __forceinline__ uint32_t spread4(uint32_t v) {
+  return (__umul24(v & 15u, 0x00204081u) & 0x01010101u) << 4;
+}
+
+constexpr float kTwo24 = 16777216.0f;  // the codes' 2^-24 is taken out in the scales
+
+// What differs between encodings.  ELEMS: elements of a unit (two blocks, or a quarter super-block); SUB: elements that share a scale;
+// MIN: whether w = scale * code + low with low != 0; chunk t of a unit is 8 elements, at chunk_at(t)
+// from the unit's first element.
+template <int TYPE>
+struct Unit {
+  static constexpr bool BLOCK32 = Block<TYPE>::QK == 32;
+  static constexpr int ELEMS = 64;
+  static constexpr int SUB = TYPE == kQ2_K || TYPE == kQ3_K || TYPE == kQ6_K ? 16 : 32;
+  static constexpr bool MIN = TYPE == kQ4_1 || TYPE == kQ5_1 || TYPE == kQ4_K || TYPE == kQ5_K || TYPE == kQ2_K;
+  static constexpr int WORDS = TYPE == kQ8_0 ? 16 : TYPE == kQ5_K || TYPE == kQ6_K || TYPE == kQ3_K ? 16 : 8;
+  // A step of four units is BYTES bytes of each row (eight blocks, or a super-block), fetched as PIECES
+  // 16-byte pieces that take ROW bytes of LDS, an odd multiple of 16 so that the lanes of a read
+  // (16 rows) start in different banks.
+  static constexpr int BYTES = BLOCK32 ? 8 * Block<TYPE>::BYTES : Block<TYPE>::BYTES;
+  static constexpr int PIECES = (BYTES + 15) / 16;
+  static constexpr int ROW = 16 * (PIECES | 1);
+  static constexpr int LOADS = (16 * PIECES + 63) / 64;  // of 16 bytes a lane, for one 16-row tile
+  uint32_t q[WORDS];  // code bytes (Q5_K, Q6_K, Q3_K: low parts, then the 8 dwords of high bits)
+  uint32_t h[4];      // scales, fifth bits and factors
+
+  // Element offset in LDS of the unit that lane group g takes of a step, from the step's first.
+  static __device__ __forceinline__ int lane_at(int g) {
+    return TYPE == kQ6_K ? 128 * (g >> 1) + 32 * (g & 1) : ELEMS * g;
+  }
+  static constexpr int chunk_at(int t) { return TYPE == kQ6_K && t >= 4 ? 64 + 8 * (t - 4) : 8 * t; }
+
+  // Read lane group g's unit from its row's pieces in LDS.
+  __device__ __forceinline__ void read(const uint8_t* row, int g) {
+    if constexpr (BLOCK32) {
+      constexpr int B = Block<TYPE>::BYTES, W = B / 2;  // dwords of two blocks
+      const uint32_t* p = reinterpret_cast<const uint32_t*>(row + 2 * B * g);
+      uint32_t v[W];
+#pragma unroll
+      for (int i = 0; i < W; ++i) v[i] = p[i];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        // dword at byte i of block b: B is even, so a block starts at byte 0 or 2 of a dword
+        auto at = [&](int i) {
+          const int byte = b * B + i;
+          return byte % 4 ? __builtin_amdgcn_alignbyte(v[byte / 4 + 1], v[byte / 4], 2) : v[byte / 4];
+        };
+        constexpr int qs = TYPE == kQ5_1 ? 8 : TYPE == kQ5_0 ? 6 : TYPE == kQ4_1 ? 4 : 2;
+        h[b] = b * B % 4 ? v[b * B / 4] >> 16 : v[b * B / 4];
+        if constexpr (MIN) h[b] = at(0);
+        if constexpr (TYPE == kQ5_0 || TYPE == kQ5_1) h[2 + b] = at(qs - 4);
+#pragma unroll
+        for (int i = 0; i < WORDS / 2; ++i) q[WORDS / 2 * b + i] = at(qs + 4 * i);
+      }
+    } else {
+      const uint8_t* p = row;
+      const int part = g;
+      const uint8_t* lo;
+      const uint8_t* hi = nullptr;
+      if constexpr (TYPE == kQ4_K || TYPE == kQ5_K) {
+        const uint4 head = *reinterpret_cast<const uint4*>(p);
+        h[0] = head.x, h[1] = head.y, h[2] = head.z, h[3] = head.w;
+        lo = p + (TYPE == kQ4_K ? 16 : 48) + 32 * part;
+        hi = p + 16;
+      } else if constexpr (TYPE == kQ6_K) {
+        lo = p + 32 * part;  // 64 h + 32 c
+        hi = p + 128 + 32 * (part >> 1);
+        const uint2 s = *reinterpret_cast<const uint2*>(p + 192 + 8 * (part >> 1));
+        h[0] = s.x, h[1] = s.y, h[2] = *reinterpret_cast<const uint16_t*>(p + 208);
+      } else if constexpr (TYPE == kQ2_K) {
+        lo = p + 16 + 32 * (part >> 1);
+        h[0] = *reinterpret_cast<const uint32_t*>(p + 4 * part);
+        h[2] = *reinterpret_cast<const uint32_t*>(p + 80);
+      } else {
+        lo = p + 32 + 32 * (part >> 1);
+        hi = p;
+        const uint4 s = *reinterpret_cast<const uint4*>(p + 96);  // 12 scale bytes, d
+        h[0] = s.x, h[1] = s.y, h[2] = s.z, h[3] = s.w & 0xFFFFu;
+      }
+      const uint4 a = *reinterpret_cast<const uint4*>(lo), b = *reinterpret_cast<const uint4*>(lo + 16);
+      q[0] = a.x, q[1] = a.y, q[2] = a.z, q[3] = a.w, q[4] = b.x, q[5] = b.y, q[6] = b.z, q[7] = b.w;
+      if constexpr (WORDS == 16) {
+        const uint4 e = *reinterpret_cast<const uint4*>(hi), f = *reinterpret_cast<const uint4*>(hi + 16);
+        q[8] = e.x, q[9] = e.y, q[10] = e.z, q[11] = e.w, q[12] = f.x, q[13] = f.y, q[14] = f.z, q[15] = f.w;
+      }
+    }
+  }
+
+  // MFMA operand of chunk t; part: the unit's index in its super-block (the lane group).
+  template <int T>
+  __device__ __forceinline__ half8_t chunk(int part) const {
+    if constexpr (TYPE == kQ8_0) {
+      return operand<128>(q[2 * T] ^ 0x80808080u, q[2 * T + 1] ^ 0x80808080u);
+    } else if constexpr (BLOCK32) {
+      constexpr int b = T >> 2, w = 4 * b + 2 * (T & 1);
+      constexpr int shift = (T & 2) ? 4 : 0;
+      uint32_t lo = (q[w] >> shift) & 0x0F0F0F0Fu, hi = (q[w + 1] >> shift) & 0x0F0F0F0Fu;
+      if constexpr (TYPE == kQ5_0 || TYPE == kQ5_1) {
+        constexpr int bit = 8 * (T & 3);  // chunk T is elements 8 (T & 3) of the block
+        lo |= spread4(h[2 + b] >> bit);
+        hi |= spread4(h[2 + b] >> (bit + 4));
+      }
+      return operand<TYPE == kQ4_0 ? 8 : TYPE == kQ5_0 ? 16 : 0>(lo, hi);
+    } else if constexpr (TYPE == kQ2_K) {
+      constexpr int w = 2 * (T & 3);
+      const int shift = 4 * (part & 1) + 2 * (T >> 2);  // plane 2 c + T / 4 of half h, part = 2 h + c
+      return operand<0>((q[w] >> shift) & 0x03030303u, (q[w + 1] >> shift) & 0x03030303u);
+    } else if constexpr (TYPE == kQ3_K) {
+      constexpr int w = 2 * (T & 3);
+      const int shift = 4 * (part & 1) + 2 * (T >> 2), bit = 2 * part + (T >> 2);
+      const uint32_t lo = ((q[w] >> shift) & 0x03030303u) | (((q[8 + w] >> bit) & 0x01010101u) << 2);
+      const uint32_t hi = ((q[w + 1] >> shift) & 0x03030303u) | (((q[9 + w] >> bit) & 0x01010101u) << 2);
+      return operand<4>(lo, hi);
+    } else {  // Q4_K, Q5_K, Q6_K: low nibbles, then high nibbles
+      constexpr int w = 2 * (T & 3), high = T >> 2;
+      uint32_t lo = (q[w] >> (4 * high)) & 0x0F0F0F0Fu, hi = (q[w + 1] >> (4 * high)) & 0x0F0F0F0Fu;
+      if constexpr (TYPE == kQ5_K) {
+        const int bit = 2 * part + high;
+        lo |= ((q[8 + w] >> bit) & 0x01010101u) << 4;
+        hi |= ((q[9 + w] >> bit) & 0x01010101u) << 4;
+      }
+      if constexpr (TYPE == kQ6_K) {
+        const int bit = 2 * (part & 1) + 4 * high;
+        lo |= ((q[8 + w] >> bit) & 0x03030303u) << 4;
+        hi |= ((q[9 + w] >> bit) & 0x03030303u) << 4;
+      }
+      return operand<TYPE == kQ6_K ? 32 : 0>(lo, hi);
+    }
+  }
+
+  // Scale (times 2^24) and low value of sub-block s of the unit, zero where the unit (or the
+  // second block of one) lies past the row's end.
+  template <int S>
+  __device__ __forceinline__ void scale(int part, bool valid, bool valid2, float& sc, float& low) const {
+    low = 0.0f;
+    if constexpr (BLOCK32) {
+      const bool in = S == 0 ? valid : valid2;
+      const uint32_t head = in ? h[S] : 0u;
+      sc = half_bits_to_float(head) * kTwo24;
+      if constexpr (MIN) low = half_bits_to_float(head >> 16);
+    } else if constexpr (TYPE == kQ4_K || TYPE == kQ5_K) {
+      const uint32_t dd = valid ? h[0] : 0u;
+      int sc_lo, mn_lo, sc_hi, mn_hi;
+      q4k_scale_pair(h[1], h[2], h[3], part, sc_lo, mn_lo, sc_hi, mn_hi);
+      sc = half_bits_to_float(dd) * (kTwo24 * (float)(S ? sc_hi : sc_lo));
+      low = -half_bits_to_float(dd >> 16) * (float)(S ? mn_hi : mn_lo);
+    } else if constexpr (TYPE == kQ6_K) {
+      // bytes 2 c, 2 c + 1 (sub-blocks 0, 1) and 2 c + 4, 2 c + 5 (2, 3) of the half's eight
+      const uint32_t pair = (S < 2 ? h[0] : h[1]) >> (16 * (part & 1));
+      const float d = half_bits_to_float(valid ? h[2] : 0u);
+      sc = d * (kTwo24 * (float)(int8_t)((pair >> (8 * (S & 1))) & 0xFFu));
+    } else if constexpr (TYPE == kQ2_K) {
+      const uint32_t dd = valid ? h[2] : 0u;
+      const uint32_t byte = h[0] >> (8 * S);
+      sc = half_bits_to_float(dd) * (kTwo24 * (float)(byte & 15u));
+      low = -half_bits_to_float(dd >> 16) * (float)((byte >> 4) & 15u);
+    } else {  // Q3_K: sub-block 4 part + S of the super-block
+      const float d = half_bits_to_float(valid ? h[3] : 0u);
+      const uint32_t nib = ((part & 1 ? h[1] : h[0]) >> (8 * S)) >> (4 * (part >> 1));
+      const uint32_t top = (h[2] >> (8 * S)) >> (2 * part);
+      sc = d * (kTwo24 * (float)((int)((nib & 15u) | ((top & 3u) << 4)) - 32));
+    }
+  }
+};
+
+// v shifted down by d bytes, zeros in from above.
+__device__ __forceinline__ uint4 shift_bytes(uint4 v, uint32_t d) {
+  if (d & 8) v = make_uint4(v.z, v.w, 0u, 0u);
+  if (d & 4) v = make_uint4(v.y, v.z, v.w, 0u);
+  const uint32_t b = d & 3u;
+  v = make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, b), __builtin_amdgcn_alignbyte(v.z, v.y, b),
+                 __builtin_amdgcn_alignbyte(v.w, v.z, b), __builtin_amdgcn_alignbyte(0u, v.w, b));
+  return d < 16u ? v : make_uint4(0u, 0u, 0u, 0u);
+}
+
+// A wave's fetch of one step of a 16-row tile: 16-byte pieces, consecutive lanes along a row.
+template <int TYPE>
+struct Fetch {
+  using U = Unit<TYPE>;
+  static constexpr int PIECES = U::PIECES;
+  const uint8_t* w;          // the tile's first row
+  uint32_t last_from;        // the largest byte offset of a piece in step 0
+  uint32_t end;              // bytes from there to the end of the matrix
+  uint32_t from[U::LOADS];   // byte offsets of the lane's pieces in step 0
+  uint32_t step_at;          // byte offset of the step in v from step 0
+  bool ragged;               // whether a piece of that step may pass the matrix's end (wave-uniform)
+  uint4 v[U::LOADS];
+
+  __device__ __forceinline__ void init(const uint8_t* matrix, int row0, int n, uint32_t row_bytes, int lane) {
+    w = matrix + (size_t)row0 * row_bytes;
+    end = (uint32_t)min((size_t)(n - row0) * row_bytes, (size_t)0xFFFFFFF0u);
+    last_from = (uint32_t)min(15, n - 1 - row0) * row_bytes + (uint32_t)(16 * (PIECES - 1));
+#pragma unroll
+    for (int i = 0; i < U::LOADS; ++i) {
+      const int piece = min(i * 64 + lane, 16 * PIECES - 1);
+      const int r = piece / PIECES, c = piece - r * PIECES;
+      from[i] = (uint32_t)min(r, n - 1 - row0) * row_bytes + (uint32_t)(16 * c);
+    }
+  }
+  // A piece that would pass the end of the matrix is read as the matrix's last 16 bytes and moved
+  // into place when it is stored (only the last tile has such pieces).
+  __device__ __forceinline__ void load(int step) {
+    step_at = (uint32_t)(step * U::BYTES);
+    ragged = last_from + step_at + 16u > end;
+#pragma unroll
+    for (int i = 0; i < U::LOADS; ++i) v[i] = load16(w + min(from[i] + step_at, end - 16u));
+  }
+  __device__ __forceinline__ void store(uint8_t* lds, int lane) {
+    if (ragged) {
+#pragma unroll
+      for (int i = 0; i < U::LOADS; ++i) {
+        const uint32_t at = from[i] + step_at;
+        v[i] = shift_bytes(v[i], at - min(at, end - 16u));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < U::LOADS; ++i) {
+      const int piece = i * 64 + lane;
+      const int r = piece / PIECES, c = piece - r * PIECES;
+      if ((i + 1) * 64 <= 16 * PIECES || piece < 16 * PIECES) *reinterpret_cast<uint4*>(lds + r * U::ROW + 16 * c) = v[i];
+    }
+  }
+};
+
+// What a launch reads besides its leading scalar arguments: the other matrices of a group and the
+// outputs.
+struct RowsMore {
+  const uint8_t* w[kGemvGroupMax - 1];  // matrices 1 and 2 (SwiGLU: up)
+  void* out[kGemvGroupMax];
+  int n[kGemvGroupMax - 1];
+  int first_block[kGemvGroupMax - 1];   // first workgroup of matrices 1 and 2
+};
+enum { kRowsHalf = 1, kRowsSwiglu = 2, kRowsGroup = 4 };  // flags
+
+// a / b for 0 <= a < 2^20 from inv = 1 / b (v_rcp_f32): an integer division costs tens of dependent
+// instructions, several of which in a row were a third of a small launch.
+__device__ __forceinline__ float inverse(int b) { return __builtin_amdgcn_rcpf((float)b); }
+__device__ __forceinline__ int quotient(int a, float inv) { return (int)(((float)a + 0.5f) * inv); }
+// The sum of v over lanes n, n + 16, n + 32 and n + 48, in each of them: the row swaps of v with
+// itself leave rows {0, 0, 2, 2} and {1, 1, 3, 3}, then rows {0, 0} and {2, 2} of the pair sums.
+__device__ __forceinline__ float sum_pieces(float v) {
+  uint32_t b = __builtin_bit_cast(uint32_t, v);
+  const auto rows = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  const uint32_t r0 = rows[0], r1 = rows[1];
+  b = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1));
+  const auto halves = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  const uint32_t h0 = halves[0], h1 = halves[1];
+  return __builtin_bit_cast(float, h0) + __builtin_bit_cast(float, h1);
+}
+__device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+constexpr int kRowsMaxK = 1 << 22;  // 16 rows stay within the 32-bit offsets of a tile
+constexpr int kRowsZero = 256;  // bytes of zeros in LDS that inactive lanes read
+
+// MR: activation rows a lane keeps sums of (1, 4 or 8).  The workgroup's waves are `per` row tiles
+// times `split` ranges of K: wave t * split + q takes steps q, q + split, .. of tile t.
+template <int TYPE, int MR>
+__global__ __launch_bounds__(768) void gemv_rows(const _Float16* __restrict__ x, const uint8_t* __restrict__ w0, int n0,
+                                                  int k, int m_rows, int per, int split, int slice_steps, int flags,
+                                                  const RowsMore more) {
+  using U = Unit<TYPE>;
+  constexpr int MG = MR > 4 ? 2 : 1;      // MFMA groups of four activation rows
+  constexpr int LIVE = MR == 1 ? 1 : 4;   // rows kept per group
+  constexpr int CHUNKS = U::ELEMS / 8, PER_SUB = U::SUB / 8, SUBS = U::ELEMS / U::SUB;
+  constexpr int XCHUNKS = MR == 1 ? 1 : MR == 4 ? 2 : 4;  // 16-byte activation chunks a thread loads at a time
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63, threads = blockDim.x;
+  const int wave = scalar(tid >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const bool pair = flags & kRowsSwiglu;
+
+  // the workgroup's matrix, the wave's row tile (SwiGLU: gate and up tiles in turn) and K range
+  const int block = blockIdx.x;
+  int mat = 0, n = n0, first_block = 0;
+  const uint8_t* w = w0;
+  if (flags & kRowsGroup) {  // (the other launches do not wait for this part of the argument block)
+    mat = (block >= more.first_block[0]) + (block >= more.first_block[1]);
+    if (mat) {
+      w = more.w[mat - 1];
+      n = more.n[mat - 1];
+      first_block = more.first_block[mat - 1];
+    }
+  }
+  const int tile_of_block = (block - first_block) * (pair ? per >> 1 : per);
+  const int tile = scalar(quotient(wave, inverse(split))), range = wave - tile * split;
+  const int blocks = k / Block<TYPE>::QK;  // of a row
+  const int units = U::BLOCK32 ? (blocks + 1) / 2 : k / U::ELEMS;
+  const int steps = (units + 3) / 4;
+  Fetch<TYPE> fetch;
+
+  // activation rows in LDS: a slice of columns each, 16 bytes past a multiple of 256 so that the
+  // rows of a b128 read start in different banks
+  const int row_lds = slice_steps * 4 * U::ELEMS * 2 + 16;
+  const int zero_at = m_rows * row_lds;
+  uint8_t* staged = lds + zero_at + kRowsZero + wave * (16 * U::ROW);  // the wave's own
+  const int xm = col & 3;
+  const bool mine = (col >> 2) == g;
+  const bool active0 = mine && xm < m_rows, active1 = MG == 2 && mine && xm + 4 < m_rows;
+  if (tid < kRowsZero / 16) *reinterpret_cast<uint4*>(lds + zero_at + 16 * tid) = make_uint4(0, 0, 0, 0);
+
+  float acc[MG][LIVE] = {};
+  half8_t ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = (_Float16)1.0f;
+
+  for (int s0 = 0; s0 < steps; s0 += slice_steps) {
+    const int last = min(s0 + slice_steps, steps);
+    const int col0 = s0 * 4 * U::ELEMS;
+    const int all16 = (last - s0) * (U::ELEMS / 2);  // 16-byte chunks of a row, with zeros to whole steps
+    const int live16 = min(all16, (k - col0) >> 3);  // those that hold activations
+    const int total = m_rows * all16;
+    const float inv16 = inverse(all16);
+    // The activations are requested first, XCHUNKS chunks a thread (past the last: the last again),
+    // then the wave's first weights, and only then are the activations waited for.
+    auto chunk_of = [&](int c, int& at, bool& live) {
+      c = min(c, total - 1);
+      const int m = quotient(c, inv16), e = c - m * all16;
+      at = m * row_lds + 16 * e;
+      live = e < live16;
+      return x + ((size_t)m * k + (uint32_t)(col0 + 8 * min(e, live16 - 1)));
+    };
+    uint4 xr[XCHUNKS];
+    int at[XCHUNKS];
+    bool live[XCHUNKS];
+#pragma unroll
+    for (int i = 0; i < XCHUNKS; ++i) xr[i] = *reinterpret_cast<const uint4*>(chunk_of(tid + i * threads, at[i], live[i]));
+    int s = s0 + range;
+    if (s0 == 0)
+      fetch.init(pair && (tile & 1) ? more.w[0] : w, min((tile_of_block + (pair ? tile >> 1 : tile)) * 16, n - 1), n,
+                 (uint32_t)(blocks * Block<TYPE>::BYTES), lane);
+    fetch.load(min(s, last - 1));
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < XCHUNKS; ++i)
+      *reinterpret_cast<uint4*>(lds + at[i]) = live[i] ? xr[i] : make_uint4(0, 0, 0, 0);
+    for (int c = tid + XCHUNKS * threads; c - tid < total; c += XCHUNKS * threads) {
+#pragma unroll
+      for (int i = 0; i < XCHUNKS; ++i) xr[i] = *reinterpret_cast<const uint4*>(chunk_of(c + i * threads, at[i], live[i]));
+#pragma unroll
+      for (int i = 0; i < XCHUNKS; ++i)
+        *reinterpret_cast<uint4*>(lds + at[i]) = live[i] ? xr[i] : make_uint4(0, 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+    for (; s < last; s += split) {
+      const int xat = ((s - s0) * 4 * U::ELEMS + U::lane_at(g)) * 2;
+      half8_t xv[CHUNKS][MG];
+      const uint8_t* x0 = lds + (active0 ? xm * row_lds + xat : zero_at);
+      const uint8_t* x1 = lds + (active1 ? (xm + 4) * row_lds + xat : zero_at);
+#pragma unroll
+      for (int t = 0; t < CHUNKS; ++t) {
+        xv[t][0] = *reinterpret_cast<const half8_t*>(x0 + 2 * U::chunk_at(t));
+        if constexpr (MG == 2) xv[t][MG - 1] = *reinterpret_cast<const half8_t*>(x1 + 2 * U::chunk_at(t));
+      }
+      U unit;
+      fetch.store(staged, lane);
+      if (s + split < last) fetch.load(s + split);
+      asm volatile("" ::: "memory");  // a wave's LDS operations complete in order
+      unit.read(staged + col * U::ROW, g);
+      asm volatile("" ::: "memory");
+      const int u = 4 * s + g;
+      const bool valid = u < units, valid2 = !U::BLOCK32 || 2 * u + 1 < blocks;
+      auto sub = [&](auto index) {
+        constexpr int S = decltype(index)::value;
+        float4v d[MG] = {}, sums[MG] = {};
+        auto mul = [&](auto offset) {
+          constexpr int T = S * PER_SUB + decltype(offset)::value;
+          const half8_t b = unit.template chunk<T>(g);
+#pragma unroll
+          for (int i = 0; i < MG; ++i) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[T][i], b, d[i], 0, 0, 0);
+          if constexpr (U::MIN) {
+#pragma unroll
+            for (int i = 0; i < MG; ++i) sums[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[T][i], ones, sums[i], 0, 0, 0);
+          }
+        };
+        mul(std::integral_constant<int, 0>{});
+        mul(std::integral_constant<int, 1>{});
+        if constexpr (PER_SUB == 4) {
+          mul(std::integral_constant<int, 2>{});
+          mul(std::integral_constant<int, 3>{});
+        }
+        float sc, low;
+        unit.template scale<S>(g, valid, valid2, sc, low);
+#pragma unroll
+        for (int i = 0; i < MG; ++i)
+#pragma unroll
+          for (int r = 0; r < LIVE; ++r) {
+            acc[i][r] = fmaf(sc, d[i][r], acc[i][r]);
+            if constexpr (U::MIN) acc[i][r] = fmaf(low, sums[i][r], acc[i][r]);
+          }
+      };
+      sub(std::integral_constant<int, 0>{});
+      sub(std::integral_constant<int, 1>{});
+      if constexpr (SUBS >= 4) {
+        sub(std::integral_constant<int, 2>{});
+        sub(std::integral_constant<int, 3>{});
+      }
+      asm volatile("" ::: "memory");
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the activations' place is free
+  }
+
+  // the four pieces' sums, then the waves' partial tiles [wave][m][16] over K in range order
+  float* partial = reinterpret_cast<float*>(lds);
+  const int tile_items = m_rows * 16;
+#pragma unroll
+  for (int i = 0; i < MG; ++i)
+#pragma unroll
+    for (int r = 0; r < LIVE; ++r) {
+      const float v = sum_pieces(acc[i][r]);
+      if (g == 0 && 4 * i + r < m_rows) partial[wave * tile_items + (4 * i + r) * 16 + col] = v;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  const int step = pair ? 2 : 1, outputs = (pair ? per >> 1 : per) * tile_items;
+  const float inv_items = inverse(tile_items);
+  for (int o = tid; o < outputs; o += threads) {
+    const int t = quotient(o, inv_items), in_tile = o - t * tile_items;
+    const float* p = partial + t * step * split * tile_items + in_tile;
+    const int row = (tile_of_block + t) * 16 + (in_tile & 15);
+    auto over_ranges = [&](const float* from) {  // in range order, four reads in flight
+      float v = 0.0f;
+      for (int q = 0; q < split; q += 4) {
+        float r[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = from[min(q + i, split - 1) * tile_items];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v += q + i < split ? r[i] : 0.0f;
+      }
+      return v;
+    };
+    float v = over_ranges(p);
+    if (pair) v = swiglu(v, over_ranges(p + split * tile_items));
+    if (row >= n) continue;
+    const size_t index = (size_t)(in_tile >> 4) * n + row;
+    if (flags & kRowsHalf) store_out(static_cast<_Float16*>(more.out[mat]), index, v);
+    else store_out(static_cast<float*>(more.out[mat]), index, v);
+  }
+}
+
+struct RowsLaunch {
+  const GemvArgs* g;
+  RowsMore more;
+  int per, split, slice_steps, flags, grid;
+  size_t lds;
+};
+
+template <int TYPE, int MR>
+hipError_t launch_rows(const RowsLaunch& l, hipStream_t stream) {
+  const GemvArgs& g = l.g[0];
+  hipLaunchKernelGGL((gemv_rows<TYPE, MR>), dim3(l.grid), dim3(64 * l.per * l.split), l.lds, stream,
+                     static_cast<const _Float16*>(g.x), static_cast<const uint8_t*>(g.w), g.n, g.k, g.m, l.per, l.split,
+                     l.slice_steps, l.flags, l.more);
+  return hipGetLastError();
+}
+
+template <int TYPE>
+hipError_t launch_rows_type(RowsLaunch& l, int count, hipStream_t stream) {
+  using U = Unit<TYPE>;
+  const int m = l.g[0].m, k = l.g[0].k;
+  const int pair = l.flags & kRowsSwiglu ? 2 : 1;  // tiles that stay together
+  int tiles = 0;
+  for (int i = 0; i < count; ++i) tiles += (l.g[i].n + 15) / 16;
+  const int steps = (k + 4 * U::ELEMS - 1) / (4 * U::ELEMS);
+  // Tiles (or pairs) per workgroup, and its waves.  Up to 1024 tiles one workgroup per CU holds them
+  // all and 12 waves (the most that leave a lane 168 registers) share their steps: 12288 x 4096 at M =
+  // 4 (768 tiles) Q4_0 9.4 us with three tiles against 10.0 with one tile and 8 waves.  Larger matrices
+  // go in workgroups of four tiles and 8 waves, two of which fit a CU beside the activations of four
+  // rows: 64000 x 4096 Q6_K at M = 4 45.6 us against 53.0 with 12 waves and 58.6 with one tile.
+  const int groups = std::max(1, std::min(tiles <= 1024 ? (tiles + 255) / 256 : 4, 12 / pair));
+  const int max_waves = tiles <= 1024 ? 12 : 8;
+  l.per = groups * pair;
+  const int most = std::max(1, std::min(max_waves / l.per, steps)), rounds = (steps + most - 1) / most;
+  l.split = (steps + rounds - 1) / rounds;  // the fewest ranges of that many steps
+  l.grid = 0;
+  for (int i = 0; i < count; ++i) {
+    l.grid += ((l.g[i].n + 15) / 16 + groups - 1) / groups;
+    if (i < kGemvGroupMax - 1) l.more.first_block[i] = i + 1 < count ? l.grid : 0x7fffffff;
+  }
+  for (int i = count; i < kGemvGroupMax - 1; ++i) l.more.first_block[i] = 0x7fffffff;
+  const int waves = l.per * l.split;
+  const int max_lds = 156 * 1024;
+  const int step_bytes = 4 * U::ELEMS * 2;
+  const int fixed = kRowsZero + 16 * m + waves * 16 * U::ROW;
+  l.slice_steps = std::max(1, std::min(steps, (max_lds - fixed) / (m * step_bytes)));
+  l.lds = std::max((size_t)m * (l.slice_steps * step_bytes) + fixed, (size_t)waves * m * 16 * 4);
+  if (m == 1) return launch_rows<TYPE, 1>(l, stream);
+  if (m <= 4) return launch_rows<TYPE, 4>(l, stream);
+  return launch_rows<TYPE, 8>(l, stream);
+}
+
+}  // namespace
+
+// Matrices of fewer elements than this (in 2^20, by activation rows 1, 2, 3, 4, more) stay on the
+// vector kernels, which reach their result sooner where latency is all: a launch of this kernel takes
+// ~1 us longer before its first product (1024 x 1024 at M = 1: Q4_0 3.0 against 2.3 us).  The lines
+// lie where graph replays of both sides crossed (shapes of 1 to 67 M elements, every encoding).
+bool gemv_rows_single(const GemvArgs& a) {
+  if (a.x_f32 || a.m < 1 || a.m > kGemvMaxM || a.k > kRowsMaxK) return false;
+  const int64_t elements = (int64_t)a.n * a.k;
+  const int at = std::min(a.m, 5) - 1;
+  auto from = [&](const int (&millions)[5]) { return elements >= (int64_t)millions[at] << 20; };
+  const bool whole_step = a.m == 1 && a.k % 4096 == 0 && a.k <= 16384;  // row lengths of the tuned M = 1 kernels
+  const bool half_step = a.m == 1 && a.k % 2048 == 0 && a.k <= 16384;
+  switch (a.type) {
+    case kQ4_0: return !half_step && from({32, 16, 3, 3, 2});
+    case kQ4_1: return !half_step && from({16, 16, 16, 6, 6});
+    case kQ5_0: return !half_step && from({16, 6, 6, 3, 6});
+    case kQ5_1: return !half_step && from({16, 16, 16, 6, 6});
+    case kQ8_0: return !half_step && from({16, 16, 6, 3, 2});
+    case kQ2_K: return !whole_step && from({16, 6, 6, 6, 6});
+    case kQ3_K: return !whole_step && from({6, 6, 3, 3, 3});
+    case kQ5_K: return !whole_step && from({6, 6, 3, 2, 2});
+    case kQ6_K: return !(whole_step && a.k <= 12288) && from({16, 2, 3, 2, 3});
+    // M > 1: the plans of tensor_gguf_gemv_plan_v1; M = 1: rows of less than 2048 columns are level
+    case kQ4_K: return a.m == 1 && !whole_step && a.k >= 2048;
+    default: return false;
+  }
+}
+
+// A group in one launch saves a launch per further matrix (q, k, v of 1024 + 2 x 128 rows and 1024
+// columns at M = 4: one launch of 3.4 us against three of 2.5 to 2.9).  Matrices that the tuned M =
+// 1 kernels stream faster each by itself keep them from 32 M elements (2 x 12288 x 4096 Q6_K: 18.4
+// against 18.9 us; 6144 x 4096 in three matrices, Q8_0: 12.4 against 8.3).
+bool gemv_rows_group(const GemvArgs* a, int count) {
+  if (count < 2 || a[0].x_f32 || a[0].m < 1 || a[0].m > kGemvMaxM || a[0].k > kRowsMaxK) return false;
+  if (a[0].m > 1 || a[0].k % 2048 != 0) return true;
+  int64_t elements = 0;
+  for (int i = 0; i < count; ++i) elements += (int64_t)a[i].n * a[i].k;
+  return elements < (int64_t)32 << 20;
+}
+
+// SwiGLU pairs: as single matrices, with the lines where the vector pair kernels (one wave per output row)
+// crossed: 2 x 3072 x 1024 at M = 2 Q8_0 4.4 against 4.9 us, at M = 4 6.1 against 5.0; 2 x 6912 x
+// 2560 at M = 1 15.4 against 11.3.  Q4_K and Q5_K at M = 1 keep their tuned row lengths; Q4_K at M > 1
+// always comes here (12288 x 4096 at M = 4 15.3 us, 18.5 on the sector kernel in pairs that this replaced).
+bool gemv_rows_pair(const GemvArgs& a) {
+  if (a.x_f32 || a.m < 1 || a.m > kGemvMaxM || a.k > kRowsMaxK) return false;
+  const bool slow = a.type == kQ3_K || a.type == kQ5_K || a.type == kQ6_K;  // pairs costly to decode per lane
+  const int millions = a.type == kQ4_K && a.m >= 2 ? 0 : a.m >= 4 || slow ? 4 : a.m == 3 ? 8 : 16;
+  if ((a.type == kQ4_K || a.type == kQ5_K) && a.m == 1 && a.k % 4096 == 0 && a.k <= 16384) return false;
+  return 2 * (int64_t)a.n * a.k >= (int64_t)millions << 20;
+}
+
+hipError_t launch_gemv_rows(const GemvArgs* g, int count, const void* w_up, hipStream_t stream) {
+  RowsLaunch l{};
+  l.g = g;
+  l.flags = (g[0].out_half ? kRowsHalf : 0) | (w_up ? kRowsSwiglu : 0) | (count > 1 ? kRowsGroup : 0);
+  for (int i = 0; i < count; ++i) {
+    l.more.out[i] = g[i].out;
+    if (i) l.more.w[i - 1] = static_cast<const uint8_t*>(g[i].w);
+    if (i) l.more.n[i - 1] = g[i].n;
+  }
+  if (w_up) l.more.w[0] = static_cast<const uint8_t*>(w_up);
+  switch (g[0].type) {
+    case kQ4_0: return launch_rows_type<kQ4_0>(l, count, stream);
+    case kQ4_1: return launch_rows_type<kQ4_1>(l, count, stream);
+    case kQ5_0: return launch_rows_type<kQ5_0>(l, count, stream);
+    case kQ5_1: return launch_rows_type<kQ5_1>(l, count, stream);
+    case kQ8_0: return launch_rows_type<kQ8_0>(l, count, stream);
+    case kQ2_K: return launch_rows_type<kQ2_K>(l, count, stream);
+    case kQ3_K: return launch_rows_type<kQ3_K>(l, count, stream);
+    case kQ4_K: return launch_rows_type<kQ4_K>(l, count, stream);
+    case kQ5_K: return launch_rows_type<kQ5_K>(l, count, stream);
+    case kQ6_K: return launch_rows_type<kQ6_K>(l, count, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace tensor_gguf

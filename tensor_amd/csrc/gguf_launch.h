@@ -48,11 +48,6 @@ hipError_t launch_gemv_q4k_fast(const GemvArgs& args, hipStream_t stream, bool* 
 bool gemv_q4k_group_supported(int m, int k, int n);
 // waves: rows (one per wave) per workgroup; 0 takes the default, 4 / 8 / 16 fix it (for sweeps)
 hipError_t launch_gemv_q4k_group(const GemvArgs* args, int count, hipStream_t stream, int waves = 0);
-// Two Q4_K matrices of one shape sharing x at 2 <= M <= 4 (K a multiple of 1024, at most 8192):
-// one launch of the sector-aligned kernel with a tile of each per workgroup; *handled is false
-// when x does not fit the kernel's LDS.
-bool gemv_q4k_pair_supported(const GemvArgs* args, int count);
-hipError_t launch_gemv_q4k_pair(const GemvArgs* args, hipStream_t stream, bool* handled);
 // Multi-row Q4_K decode GEMV plans (2 <= M <= 8, fp16 x): the kernel and its launch shape.
 //   kGemvSec  (gemv_q4k_sec):  a = 16-row tiles per workgroup (1-3), b = 1 to stage x before
 //                              the weight loads are issued, 0 to issue them behind x
@@ -82,8 +77,8 @@ hipError_t launch_gemv_q8_1(const GemvArgs& args, hipStream_t stream);
 // Decode GEMV with the SwiGLU epilogue of an MLP: out = silu(x W_gate^T) * (x W_up^T),
 // args.w the gate matrix, w_up the up matrix of the same shape and encoding.
 hipError_t launch_gemv_swiglu(const GemvArgs& gate, const void* w_up, hipStream_t stream);
-// Its fast paths: Q4_K / Q5_K at M = 1 (gate and up rows of one workgroup; waves: 8 or 16 per
-// workgroup, 0 the default) and Q4_K at 2 <= M <= 8 (a gate tile and its up tile per workgroup).
+// Its fast path: Q4_K / Q5_K at M = 1 (gate and up rows of one workgroup; waves: 8 or 16 per
+// workgroup, 0 the default).
 hipError_t launch_gemv_q4k_swiglu_fast(const GemvArgs& gate, const void* w_up, hipStream_t stream, bool* handled,
                                        int waves = 0);
 // fp32-activation fast path at M = 1 for Q4_K and Q5_K (K a multiple of 4096, at most 16384);
@@ -97,6 +92,14 @@ hipError_t launch_gemv_q5k_fast(const GemvArgs& args, hipStream_t stream, bool* 
 hipError_t launch_gemv_q6k_fast(const GemvArgs& args, hipStream_t stream, bool* handled);
 // Q2_K / Q3_K fast path (LDS-staged x, per-sub-block decode, M = 1, K in {4096, 8192, 12288, 16384}).
 hipError_t launch_gemv_q23k_fast(const GemvArgs& args, hipStream_t stream, bool* handled);
+// Decode GEMV on matrix cores, every encoding and K, fp16 x: `count` matrices that share x, or
+// (w_up set, count 1) the SwiGLU pair.
+hipError_t launch_gemv_rows(const GemvArgs* args, int count, const void* w_up, hipStream_t stream);
+// Whether it is the better kernel for a single matrix, a group (args of one x, K, encoding and output
+// type) and a SwiGLU pair of matrices like a.
+bool gemv_rows_single(const GemvArgs& a);
+bool gemv_rows_group(const GemvArgs* args, int count);
+bool gemv_rows_pair(const GemvArgs& a);
 hipError_t launch_dequant(const DequantArgs& args, hipStream_t stream);
 hipError_t launch_gemm(const GemvArgs& args, hipStream_t stream);
 
