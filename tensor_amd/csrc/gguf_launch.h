@@ -142,6 +142,12 @@ bool gemm_group_pipelined(const GemmGroupArgs& args, const GemmPlan& plan);
 // workspace is short.  A split plan also launches the in-order reduction of the partial sums.
 hipError_t launch_gemm_group_plan(const GemmGroupArgs& args, const GemmPlan& plan, void* workspace,
                                   size_t workspace_bytes, hipStream_t stream);
+// The encodings without plans (Q4_1, Q5_0, Q5_1, Q2_K, Q3_K; fp16 x) on the pipelined kernel, unsplit:
+// whether it covers the group, its launch, and the launch on a given tile.
+bool gemm_more_type(int type);
+bool gemm_group_more(const GemmGroupArgs& args);
+hipError_t launch_gemm_group_more(const GemmGroupArgs& args, hipStream_t stream);
+hipError_t launch_gemm_pipe_more(const GemmGroupArgs& args, int tile, hipStream_t stream);
 // Whether the pipelined kernel covers this single-matrix shape (as launch_gemm_pipe runs it).
 bool gemm_pipe_supported(const GemvArgs& args);
 // Pipelined dequant-GEMM of one matrix; sets *handled to false for the encodings and shapes it

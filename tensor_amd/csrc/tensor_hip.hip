@@ -624,6 +624,8 @@ int32_t gemm_group_call(const TensorCallV1* call, TensorErrorV1* error, bool has
   }
   if ((!small || plan.small_m) && tensor_gguf::gemm_group_pipelined(group, plan)) {
     status = tensor_gguf::launch_gemm_group_plan(group, plan, workspace, workspace_bytes, stream);
+  } else if (!small && tensor_gguf::gemm_group_more(group)) {
+    status = tensor_gguf::launch_gemm_group_more(group, stream);
   } else {
     // the other encodings and shapes, and small M where the plan keeps the small-M kernel, one
     // launch per matrix in order (no workspace: such plans never split K)
