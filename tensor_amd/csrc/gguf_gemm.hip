@@ -214,22 +214,17 @@ static hipError_t launch_tile(const GemvArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The small-M kernel where the tiled kernels leave most CUs idle: M <= 64 for shapes on the
-// generic tiles, and for shapes the pipelined tiles take also N <= 4096 (at N = 12288 those are
-// faster from M = 16: Q4_K M = 32, K = 4096: 33.6 against 38.4 us, Q4_0 with fp16 x 23.4
-// against 40.9; at N = K = 1024, M = 32 the small-M kernel takes 5.3 against 10.4 us, Q4_0
-// 4.9 against 30.6).  Q8_0 with fp32 x keeps it to M = 16 (33.7 against 42.8 us at N = 12288).
-// The encodings without plans (Q4_1, Q5_0, Q5_1, Q2_K, Q3_K) keep it below 32 M elements too: 6912 x
-// 2560 at M = 16 / 64 Q4_1 12.3 / 20.6 against 20.9 / 22.4 us, Q3_K 22.2 / 20.1 against 22.8 /
-// 24.0, while 12288 x 4096 takes 27.1 / 45.7 against 24.6 / 27.4 and 42.8 / 51.4 against 33.1 / 35.7.
+// The small-M kernel where the streaming kernel (gemm_rows_takes) leaves a call to it or a plan asks: M <= 64
+// for shapes on the generic tiles, and for shapes the pipelined tiles take also N <= 4096.
 bool gemm_small_m(const GemvArgs& a) {
   if (!gemm_skinny_supported(a)) return false;
-  if (gemm_more_type(a.type)) return !gemm_pipe_supported(a) || a.n <= 4096 || (int64_t)a.n * a.k < (int64_t)32 << 20;
   return !gemm_pipe_supported(a) || a.n <= 4096 || (a.type == kQ8_0 && a.x_f32 && a.m <= 16);
 }
 
 template <int TYPE, typename OutT>
 static hipError_t launch_type(const GemvArgs& a, hipStream_t stream) {
+  const GemmGroupArgs group = gemm_single(a);
+  if (gemm_rows_takes(group, GemmPlan{0, 1})) return launch_gemm_rows(group, stream);
   if (gemm_small_m(a)) return launch_gemm_skinny(a, stream);
   bool handled = false;
   const hipError_t status = launch_gemm_pipe(a, stream, &handled);

@@ -206,7 +206,7 @@ bool gemm_group_pipelined(const GemmGroupArgs& a, const GemmPlan& plan) {
   return pipe_type(a.type) && valid_plan(a, plan.tile, plan.splits);
 }
 
-static GemmGroupArgs single(const GemvArgs& a) {
+GemmGroupArgs gemm_single(const GemvArgs& a) {
   GemmGroupArgs g{};
   g.x = a.x;
   g.w[0] = a.w;
@@ -223,7 +223,7 @@ static GemmGroupArgs single(const GemvArgs& a) {
 
 hipError_t launch_gemm_pipe_config(const GemvArgs& a, hipStream_t stream, int config) {
   if (a.x_f32 || !pipe_type(a.type)) return hipErrorInvalidValue;
-  return launch_gemm_group_plan(single(a), GemmPlan{config, 1}, nullptr, 0, stream);
+  return launch_gemm_group_plan(gemm_single(a), GemmPlan{config, 1}, nullptr, 0, stream);
 }
 
 // Q4_1, Q5_0, Q5_1, Q2_K and Q3_K with fp16 x, on the tile an unsplit plan would take: no K split across
@@ -245,12 +245,12 @@ hipError_t launch_gemm_group_more(const GemmGroupArgs& a, hipStream_t stream) {
 }
 
 bool gemm_pipe_supported(const GemvArgs& a) {
-  const GemmGroupArgs g = single(a);
+  const GemmGroupArgs g = gemm_single(a);
   return gemm_group_pipelined(g, plan_gemm_group(g, 0)) || gemm_group_more(g);
 }
 
 hipError_t launch_gemm_pipe(const GemvArgs& a, hipStream_t stream, bool* handled) {
-  const GemmGroupArgs g = single(a);
+  const GemmGroupArgs g = gemm_single(a);
   const GemmPlan plan = plan_gemm_group(g, 0);
   if (gemm_group_more(g)) {
     *handled = true;

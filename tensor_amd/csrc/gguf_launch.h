@@ -164,6 +164,12 @@ hipError_t launch_gemm_pipe_config(const GemvArgs& args, hipStream_t stream, int
 constexpr int kSkinnyMaxM = 64;
 bool gemm_skinny_supported(const GemvArgs& args);
 hipError_t launch_gemm_skinny(const GemvArgs& args, hipStream_t stream, int nt = 0, int mt = 0);
+// Dequant-GEMM of up to 64 activation rows that streams the weights, every encoding: a group of
+// matrices in one launch; whether it takes the group from the plan given.
+bool gemm_rows_takes(const GemmGroupArgs& args, const GemmPlan& plan);
+hipError_t launch_gemm_rows(const GemmGroupArgs& args, hipStream_t stream);
+// One matrix as a group.
+GemmGroupArgs gemm_single(const GemvArgs& args);
 // Whether launch_gemm takes the small-M kernel for this shape.
 bool gemm_small_m(const GemvArgs& args);
 

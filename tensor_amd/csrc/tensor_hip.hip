@@ -603,8 +603,9 @@ int32_t gemm_group_call(const TensorCallV1* call, TensorErrorV1* error, bool has
   }
   if (int32_t s = check_device(call, error)) return s;
   hipStream_t stream = reinterpret_cast<hipStream_t>(call->stream.handle);
+  const bool rows = !forced && tensor_gguf::gemm_rows_takes(group, plan);
   ScratchLease lease;
-  if (!has_workspace) {
+  if (!has_workspace && !rows) {
     if (int32_t s = lease.acquire(call, stream, error)) return s;
     workspace = lease.address();
   }
@@ -622,7 +623,9 @@ int32_t gemm_group_call(const TensorCallV1* call, TensorErrorV1* error, bool has
     one[i].out_half = group.out_half;
     small = small && tensor_gguf::gemm_small_m(one[i]);
   }
-  if ((!small || plan.small_m) && tensor_gguf::gemm_group_pipelined(group, plan)) {
+  if (rows) {
+    status = tensor_gguf::launch_gemm_rows(group, stream);
+  } else if ((!small || plan.small_m) && tensor_gguf::gemm_group_pipelined(group, plan)) {
     status = tensor_gguf::launch_gemm_group_plan(group, plan, workspace, workspace_bytes, stream);
   } else if (!small && tensor_gguf::gemm_group_more(group)) {
     status = tensor_gguf::launch_gemm_group_more(group, stream);
@@ -632,7 +635,7 @@ int32_t gemm_group_call(const TensorCallV1* call, TensorErrorV1* error, bool has
     for (int i = 0; i < count && status == hipSuccess; ++i) status = tensor_gguf::launch_gemm(one[i], stream);
   }
   if (status != hipSuccess) return hip_fail(error, status, "GGUF grouped GEMM launch");
-  return has_workspace ? TENSOR_OK : lease.release(stream, error);
+  return has_workspace || rows ? TENSOR_OK : lease.release(stream, error);
 }
 
 }  // namespace
