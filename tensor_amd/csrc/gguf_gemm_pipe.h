@@ -473,26 +473,47 @@ __global__ __launch_bounds__(WM * WN * 64 * KS) void gemm_pipe(const XT* __restr
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
 
+  // fragments of one 32-wide half kk of the step staged in (xs, ws)
+  auto fragments = [&](half8_t (&a)[MT], half8_t (&b)[NT], const _Float16* xs, const _Float16* ws, int kk) {
+    const int koff = 32 * kk + 8 * (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int row = wm + 16 * i + (lane & 15);
+      if constexpr (XDMA)
+        a[i] = *reinterpret_cast<const half8_t*>(&xs[row * BK + 8 * ((4 * kk + (lane >> 4)) ^ ((row >> 1) & 7))]);
+      else
+        a[i] = *reinterpret_cast<const half8_t*>(&xs[row * ROW + koff]);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      b[j] = *reinterpret_cast<const half8_t*>(&ws[(wn + 16 * j + (lane & 15)) * ROW + koff]);
+  };
+  auto multiply = [&](const half8_t (&a)[MT], const half8_t (&b)[NT]) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], acc[i][j], 0, 0, 0);
+  };
+  // XDMA: the fragments of the last step's second half, multiplied first in the next: the matrix
+  // pipe has work while that step's fragments come from LDS (without it and with x through registers,
+  // a 256 x 128 step took 2700 cycles for 1024 of MFMA work).  M = 2048: Q6_K 4096 x 12288
+  // 274 -> 251 us, Q8_0 269 -> 219, Q4_K 4096 x 4096 80 -> 77, Q5_K 99 -> 81, Q3_K 143 -> 88; the
+  // 256 x 192 tile 395 -> 389 (Q4_K 24576 x 4096).  Weights two steps ahead measured no faster.
+  half8_t a1[MT], b1[NT];
+  if constexpr (XDMA) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) a1[i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < NT; ++j) b1[j] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+  }
+
   // one K step: fragment reads of (xs, ws), then MFMAs interleaved with the
   // staging of `staged` into (xn, wnext) and the prefetch of `fetch_step`
   auto step_body = [&](const _Float16* xs, const _Float16* ws, _Float16* xn, _Float16* wnext, const RawT& staged,
                        int staged_step, RawT& fetched, int fetch_step, _Float16* xdma = nullptr) {
     half8_t a[2][MT], b[2][NT];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      const int koff = 32 * kk + 8 * (lane >> 4);
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int row = wm + 16 * i + (lane & 15);
-        if constexpr (XDMA)
-          a[kk][i] = *reinterpret_cast<const half8_t*>(&xs[row * BK + 8 * ((4 * kk + (lane >> 4)) ^ ((row >> 1) & 7))]);
-        else
-          a[kk][i] = *reinterpret_cast<const half8_t*>(&xs[row * ROW + koff]);
-      }
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-        b[kk][j] = *reinterpret_cast<const half8_t*>(&ws[(wn + 16 * j + (lane & 15)) * ROW + koff]);
-    }
+    fragments(a[0], b[0], xs, ws, 0);
     if constexpr (XDMA) {
       // the x DMA of the fetched step is issued ahead of its weight loads and the order is pinned:
       // loads complete in order, so once a wave's dequant has waited on those weights (the next
@@ -501,13 +522,10 @@ __global__ __launch_bounds__(WM * WN * 64 * KS) void gemm_pipe(const XT* __restr
       // they dequantize, the lower half (two parts) after, so the two waves that share a SIMD
       // keep its matrix pipe and its VALU busy at the same time.
       auto mfma_all = [&]() {
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-          for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[kk][i], b[kk][j], acc[i][j], 0, 0, 0);
+        multiply(a1, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        fragments(a1, b1, xs, ws, 1);
+        multiply(a[0], b[0]);
       };
       const bool mfma_first = wave >= WM * WN / 2;
       if (mfma_first) {
@@ -525,6 +543,7 @@ __global__ __launch_bounds__(WM * WN * 64 * KS) void gemm_pipe(const XT* __restr
       }
       return;
     }
+    fragments(a[1], b[1], xs, ws, 1);
     store(staged, xn, wnext, staged_step);
     load(fetched, fetch_step);
 #pragma unroll
@@ -573,6 +592,7 @@ __global__ __launch_bounds__(WM * WN * 64 * KS) void gemm_pipe(const XT* __restr
       __builtin_amdgcn_sched_barrier(0);
       cur = c2;
     }
+    multiply(a1, b1);
   } else {
     load(ra, first);
     load(rb, first + 1);
@@ -756,7 +776,7 @@ hipError_t launch_pipe(const GemmGroupArgs& a, int splits, void* workspace, hipS
 template <int TYPE, typename OutT, typename XT>
 hipError_t launch_tile(const GemmGroupArgs& a, int tile, int splits, void* workspace, hipStream_t stream) {
   switch (tile) {
-    case 0: return launch_pipe<TYPE, 256, 128, 4, 2, 1, OutT, XT>(a, splits, workspace, stream);
+    case 0: return launch_pipe<TYPE, 256, 128, 4, 2, 1, OutT, XT, sizeof(XT) == 2>(a, splits, workspace, stream);
     case 1: return launch_pipe<TYPE, 128, 128, 2, 2, 1, OutT, XT>(a, splits, workspace, stream);
     case 2: return launch_pipe<TYPE, 128, 64, 2, 2, 1, OutT, XT>(a, splits, workspace, stream);
     case 3: return launch_pipe<TYPE, 64, 64, 1, 2, 1, OutT, XT>(a, splits, workspace, stream);

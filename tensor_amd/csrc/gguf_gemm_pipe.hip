@@ -16,11 +16,12 @@
 //   * each step is one straight-line region in which sched_group_barrier
 //     interleaves every MFMA with dequant VALU work, an LDS store or a global
 //     load, keeping the matrix pipe fed while the VALU decodes;
-//   * XDMA (the 256 x 192 tile): the activation tile goes from global memory
-//     straight to LDS (global_load_lds_dwordx4, three swizzled buffers), which
-//     frees the staging registers the wider tile needs; half of its waves issue
-//     a step's MFMAs before their dequant and half after, so the two waves of a
-//     SIMD overlap matrix and vector work (ping-pong);
+//   * XDMA (the 256 x 192 tile, and 256 x 128 with fp16 x): the activation tile
+//     goes from global memory straight to LDS (global_load_lds_dwordx4, three
+//     swizzled buffers), which frees the staging registers the wider tile needs;
+//     half of its waves issue a step's MFMAs before their dequant and half after,
+//     so the two waves of a SIMD overlap matrix and vector work (ping-pong), and
+//     the MFMAs of a step's second half run under the next step's LDS reads;
 //   * Q4_K / Q5_K with four (two) threads per weight row: the lanes of a row, a
 //     DPP quad (pair), each decode one (two) of the step's four scale factors
 //     and share them by broadcasts, instead of each decoding all four.
@@ -102,6 +103,9 @@ constexpr long kMinBlocks = 160;
 // + up at M = 256 (192 -> 256 workgroups, one round): 70.9 -> 64.9 us and 71.1 -> 64.6 us; Q6_K
 // and Q8_0 at C4 M = 512 88.4 -> 79.9 and 79.2 -> 67.0 us; at M = 2048 (three rounds against
 // four) the 128-column tile stays (229.7 against 257.4 us).
+//
+// (With x by LDS DMA in the 256 x 128 tile too its steps came down, Q4_K 4096 x 4096 at M = 2048
+// from 1.25 to 1.20 us; the lines between the tiles stay where they were.)
 //
 // 256 x 192 (x by LDS DMA, ping-pong waves) steps take 1.3 of a 256 x 128 step and 1.5 of a
 // 256 x 96 one (Q4_K, timing harness: 1.50-1.54 against 1.12 and 0.97-0.99 us per step at
