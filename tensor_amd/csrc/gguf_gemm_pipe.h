@@ -122,7 +122,7 @@ struct Raw {
 
 }  // namespace pipe
 
-// KS groups of WM x WN waves split K: group g takes steps [g S, g S + S), S = steps / KS,
+// KS groups of WM x WN waves split K: each takes a run of steps (equal but for a unit of two or four)
 // with its own LDS staging buffers; the KS partial tiles are summed in LDS at the end
 // (KS = 1: the whole K range in one group).
 //
@@ -188,10 +188,13 @@ __global__ __launch_bounds__(WM * WN * 64 * KS) void gemm_pipe(const XT* __restr
     wpart[p] = part % TPR;
     wbase[p] = (uint32_t)min(n0 + wrow[p], N - 1) * (uint32_t)((K / QK) * BYTES);
   }
-  // this group's steps of this split; the host guarantees that every group takes an even number
-  // of steps and (for the 256-element encodings) starts on a super-block
-  const int split_steps = K / BK / job.splits;
-  const int steps = split_steps / KS, first = blockIdx.z * split_steps + group * steps;
+  // this group's steps of this split, in units of two (a super-block's four for the 256-element
+  // encodings), which the first groups take one more of where they don't divide evenly; the host
+  // guarantees whole units and one for every group
+  constexpr int UNIT = B32 ? 2 : 4;
+  const int split_steps = K / BK / job.splits, units = split_steps / UNIT, more = units % KS;
+  const int steps = UNIT * (units / KS + (group < more ? 1 : 0));
+  const int first = blockIdx.z * split_steps + UNIT * (group * (units / KS) + min(group, more));
 
   // XDMA: DMA source rows of this lane.  Block b = XPW wave + i of the x tile (1 KB, 8 rows of
   // 128 B) goes to LDS lane-linear: lane l writes 16 B at 16 l, row 8 b + l / 8, slot l % 8, which
@@ -604,6 +607,11 @@ __global__ __launch_bounds__(WM * WN * 64 * KS) void gemm_pipe(const XT* __restr
       __syncthreads();
       step_body(xs1, ws1, xs0, ws0, ra, min(step + 2, last), rb, min(step + 3, last));
       __syncthreads();
+    }
+    if constexpr (KS > 1) {
+      // the barriers of the groups that took a unit more
+      if (more > 0 && group >= more)
+        for (int i = 0; i < UNIT; ++i) __syncthreads();
     }
   }
   if constexpr (KS > 1) {

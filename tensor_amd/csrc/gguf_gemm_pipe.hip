@@ -121,9 +121,11 @@ int wide_tile(const GemmGroupArgs& a) {
   return rounds(8) * 84 < rounds(0) * 100 ? 8 : 0;
 }
 
-int base_tile(const GemmGroupArgs& a) {
+// uneven: wave groups may take unequal shares of K.
+int base_tile(const GemmGroupArgs& a, bool uneven = false) {
   const int steps = a.k / pipe::BK;  // even (whole 32-element block pairs or super-blocks)
-  const bool ks2 = steps % 8 == 0, ks4 = steps % 16 == 0;
+  const int units = steps / (block32(a.type) ? 2 : 4);
+  const bool ks2 = uneven ? units >= 2 : steps % 8 == 0, ks4 = uneven ? units >= 4 : steps % 16 == 0;
   if (a.m > 128 && tile_count(a, kTiles[0]) >= kMinBlocks) return wide_tile(a);
   if (a.m > 64) {
     const long wide = tile_count(a, kTiles[1]);
@@ -239,13 +241,16 @@ bool gemm_more_type(int type) {
   return type == kQ4_1 || type == kQ5_0 || type == kQ5_1 || type == kQ2_K || type == kQ3_K;
 }
 
+// No plan names their tiles, so the wave groups of a workgroup may share K unevenly, which K = 2560 (40
+// steps) and 6912 (108) otherwise rule out.  Q3_K at M = 333 on 64 x 64 tiles: 2560 x 6912 94 us in one
+// group -> 56 in four, 2560 x 2560 24.3 in two -> 22.9 in four.
 bool gemm_group_more(const GemmGroupArgs& a) {
-  return gemm_more_type(a.type) && !a.x_f32 && valid_plan(a, base_tile(a), 1);
+  return gemm_more_type(a.type) && !a.x_f32 && valid_plan(a, 3, 1);  // base_tile picks no more groups than K has units
 }
 
 hipError_t launch_gemm_group_more(const GemmGroupArgs& a, hipStream_t stream) {
   if (!gemm_group_more(a) || a.count < 1 || a.count > kGemmGroupMax) return hipErrorInvalidValue;
-  return launch_gemm_pipe_more(a, base_tile(a), stream);
+  return launch_gemm_pipe_more(a, base_tile(a, true), stream);
 }
 
 bool gemm_pipe_supported(const GemvArgs& a) {

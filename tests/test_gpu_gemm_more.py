@@ -63,3 +63,19 @@ def test_tiles_against_the_prefill_numerics(hip_device, encoding, m, k, rows):
         bound = k * 2.0 ** -24 * (np.abs(xd) @ np.abs(w).T) + 1e-12
         assert not np.isnan(got).any()
         assert (np.abs(got - xd @ w.T) <= bound).all()
+
+
+@pytest.mark.parametrize("encoding", ENCODINGS)
+@pytest.mark.parametrize("units", [2, 3, 5, 7])  # K in pairs of steps or super-blocks: shares of 1-2 over 2 or 4 wave groups
+def test_uneven_shares_of_k(hip_device, encoding, units):
+    k = units * (128 if Q.GEOMETRY[Q.ggml_type(encoding)][0] == 32 else 256)
+    for m, rows in ((100, (70, 33)), (333, (2560,)), (140, (12000,))):
+        print("[gemm-more] uneven", encoding, m, k, rows, flush=True)
+        x = cases.activation(m, k, 95)
+        raws = [cases.weight(n, k, encoding, 96 + i) for i, n in enumerate(rows)]
+        for got, raw, n in zip(group(hip_device, encoding, x, raws), raws, rows):
+            w = R.dequantize(raw, Q.ggml_type(encoding), n, k).astype(np.float16).astype(np.float64)
+            xd = x.astype(np.float64)
+            bound = k * 2.0 ** -24 * (np.abs(xd) @ np.abs(w).T) + 1e-12
+            assert not np.isnan(got).any()
+            assert (np.abs(got - xd @ w.T) <= bound).all(), (encoding, m, n, k)
