@@ -5,7 +5,7 @@
 // The fetch of the matrix-core decode GEMV (gguf_gemv_rows.hip): a wave takes 16 rows x 256 columns at a
 // time, 16-byte pieces along the rows, passed through LDS to the lanes that own them (lane n + 16 g:
 // unit g of row n).  A lane turns each 8 codes of its unit into fp16 weights (one fp32 fma per code from
-// its exact subnormal, then the fp16 cast: the values every GEMM here stages) and they are
+// its exact fp16 value, then the fp16 cast: the values every GEMM here stages) and they are
 // the B operand of one MFMA per 16 activation rows as they are: the A operand's lane m + 16 g reads
 // x[m] at the columns of unit g, so any assignment of columns to lane groups gives the same sum.
 // Weights go through no LDS tile after decoding and are decoded once for all M.

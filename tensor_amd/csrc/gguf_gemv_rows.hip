@@ -14,9 +14,9 @@
 // ~60 of the decode (M > 4 takes a second MFMA for rows 4..7), while a vector dot product
 // would spend M / 2 instructions per weight pair and read M activations per weight from LDS.
 //
-// Codes enter the MFMA as fp16 subnormals (code * 2^-24: v_perm_b32 widens bytes with a zero
-// high byte; the MFMA keeps subnormals), so nothing is biased and cancelled; encodings with a
-// constant offset subtract it exactly (v_pk_add_f16).  Minimums multiply the sums of x over their
+// Codes enter the MFMA as fp16 code * 2^-9 (v_perm_b32 widens bytes with a zero high byte, one packed
+// multiply, or a fma that subtracts a constant offset exactly, makes the subnormal normal), so
+// nothing is biased and cancelled.  Minimums multiply the sums of x over their
 // 16 or 32 elements, which come from an MFMA of the same activations with ones.
 //
 // A workgroup owns one or a few 16-row tiles and splits K over its waves; a wave fetches 16 rows x 256
@@ -347,7 +347,7 @@ bool gemv_rows_group(const GemvArgs* a, int count) {
 // SwiGLU pairs: as single matrices, with the lines where the vector pair kernels (one wave per output row)
 // crossed: 2 x 3072 x 1024 at M = 2 Q8_0 4.4 against 4.9 us, at M = 4 6.1 against 5.0; 2 x 6912 x
 // 2560 at M = 1 15.4 against 11.3.  Q4_K and Q5_K at M = 1 keep their tuned row lengths; Q4_K at M > 1
-// always comes here (12288 x 4096 at M = 4 15.3 us, 18.5 on the sector kernel in pairs that this replaced).
+// always comes here (12288 x 4096 at M = 4 about 16 us, 18.5 on the sector kernel in pairs that this replaced).
 bool gemv_rows_pair(const GemvArgs& a) {
   if (a.x_f32 || a.m < 1 || a.m > kGemvMaxM || a.k > kRowsMaxK) return false;
   const bool slow = a.type == kQ3_K || a.type == kQ5_K || a.type == kQ6_K;  // pairs costly to decode per lane

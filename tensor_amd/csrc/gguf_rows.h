@@ -15,14 +15,20 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint32_t sub01(uint32_t c) { return __builtin_amdgcn_perm(0u, c, 0x0C010C00u); }
 __device__ __forceinline__ uint32_t sub23(uint32_t c) { return __builtin_amdgcn_perm(0u, c, 0x0C030C02u); }
 
-// The eight byte codes of two dwords as an MFMA operand, OFFSET (< 1024) subtracted from each.
+// The eight byte codes of two dwords less OFFSET as an MFMA operand, times 2^-9.  The subnormals are
+// made normal (exact: v_pk_fma_f16, or v_pk_mul_f16 without an offset) since the MFMA aligns a
+// product by its operands' exponent fields: with the codes left at 2^-24 its sums lost as many bits
+// as the codes have leading zeros (8192 x 2560 fp32 sums against fp64: Q2_K 8.9e-6, Q4_1 4.9e-6, Q8_0 3.4e-7;
+// normal, all encodings: 0.7e-7 to 1.0e-7, for 3-4% of a Q4_K layer's time).
 template <int OFFSET>
 __device__ __forceinline__ half8_t operand(uint32_t lo, uint32_t hi) {
   uint32_t v[4] = {sub01(lo), sub23(lo), sub01(hi), sub23(hi)};
-  if constexpr (OFFSET != 0) {
-    constexpr uint32_t off = 0x80008000u | (uint32_t)OFFSET | ((uint32_t)OFFSET << 16);
+  const half2_t up = {(_Float16)32768.0f, (_Float16)32768.0f};
+  const half2_t off = {(_Float16)(-OFFSET / 512.0f), (_Float16)(-OFFSET / 512.0f)};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = __builtin_bit_cast(uint32_t, as_half2(v[i]) + as_half2(off));
+  for (int i = 0; i < 4; ++i) {
+    const half2_t c = as_half2(v[i]);
+    v[i] = __builtin_bit_cast(uint32_t, OFFSET != 0 ? __builtin_elementwise_fma(c, up, off) : c * up);
   }
   return __builtin_bit_cast(half8_t, make_uint4(v[0], v[1], v[2], v[3]));
 }
@@ -32,7 +38,7 @@ __device__ __forceinline__ uint32_t spread4(uint32_t v) {
   return (__umul24(v & 15u, 0x00204081u) & 0x01010101u) << 4;
 }
 
-constexpr float kTwo24 = 16777216.0f;  // the codes' 2^-24 is taken out in the scales
+constexpr float kTwo9 = 512.0f;  // the codes' 2^-9 is taken out in the scales
 
 // What differs between encodings.  ELEMS: elements of a unit (two blocks, or a quarter super-block); SUB: elements that share a scale;
 // MIN: whether w = scale * code + low with low != 0; chunk t of a unit is 8 elements, at chunk_at(t)
@@ -158,7 +164,7 @@ struct Unit {
     }
   }
 
-  // Scale (times 2^24) and low value of sub-block s of the unit, zero where the unit (or the
+  // Scale (times 2^9) and low value of sub-block s of the unit, zero where the unit (or the
   // second block of one) lies past the row's end.
   template <int S>
   __device__ __forceinline__ void scale(int part, bool valid, bool valid2, float& sc, float& low) const {
@@ -166,29 +172,29 @@ struct Unit {
     if constexpr (BLOCK32) {
       const bool in = S == 0 ? valid : valid2;
       const uint32_t head = in ? h[S] : 0u;
-      sc = half_bits_to_float(head) * kTwo24;
+      sc = half_bits_to_float(head) * kTwo9;
       if constexpr (MIN) low = half_bits_to_float(head >> 16);
     } else if constexpr (TYPE == kQ4_K || TYPE == kQ5_K) {
       const uint32_t dd = valid ? h[0] : 0u;
       int sc_lo, mn_lo, sc_hi, mn_hi;
       q4k_scale_pair(h[1], h[2], h[3], part, sc_lo, mn_lo, sc_hi, mn_hi);
-      sc = half_bits_to_float(dd) * (kTwo24 * (float)(S ? sc_hi : sc_lo));
+      sc = half_bits_to_float(dd) * (kTwo9 * (float)(S ? sc_hi : sc_lo));
       low = -half_bits_to_float(dd >> 16) * (float)(S ? mn_hi : mn_lo);
     } else if constexpr (TYPE == kQ6_K) {
       // bytes 2 c, 2 c + 1 (sub-blocks 0, 1) and 2 c + 4, 2 c + 5 (2, 3) of the half's eight
       const uint32_t pair = (S < 2 ? h[0] : h[1]) >> (16 * (part & 1));
       const float d = half_bits_to_float(valid ? h[2] : 0u);
-      sc = d * (kTwo24 * (float)(int8_t)((pair >> (8 * (S & 1))) & 0xFFu));
+      sc = d * (kTwo9 * (float)(int8_t)((pair >> (8 * (S & 1))) & 0xFFu));
     } else if constexpr (TYPE == kQ2_K) {
       const uint32_t dd = valid ? h[2] : 0u;
       const uint32_t byte = h[0] >> (8 * S);
-      sc = half_bits_to_float(dd) * (kTwo24 * (float)(byte & 15u));
+      sc = half_bits_to_float(dd) * (kTwo9 * (float)(byte & 15u));
       low = -half_bits_to_float(dd >> 16) * (float)((byte >> 4) & 15u);
     } else {  // Q3_K: sub-block 4 part + S of the super-block
       const float d = half_bits_to_float(valid ? h[3] : 0u);
       const uint32_t nib = ((part & 1 ? h[1] : h[0]) >> (8 * S)) >> (4 * (part >> 1));
       const uint32_t top = (h[2] >> (8 * S)) >> (2 * part);
-      sc = d * (kTwo24 * (float)((int)((nib & 15u) | ((top & 3u) << 4)) - 32));
+      sc = d * (kTwo9 * (float)((int)((nib & 15u) | ((top & 3u) << 4)) - 32));
     }
   }
 };

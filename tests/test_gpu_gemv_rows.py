@@ -116,3 +116,17 @@ def test_swiglu_pairs(hip_device, encoding, m, n, k):
     assert not np.isnan(got).any()
     assert (np.abs(got - want) <= 1.2 * eg * np.abs(u) + 1.2 * eu * np.abs(R.silu(g)) + 2 * eg * eu
             + 1e-5 * np.abs(want) + 1e-9).all()
+
+
+@pytest.mark.parametrize("encoding", ENCODINGS)
+def test_sums_keep_fp32_precision(hip_device, encoding):
+    """Against fp64 over all outputs: each rounds a few dozen times by at most 2^-24 of a partial sum,
+    errors of independent signs (random activations), so 2^-20 relative L2 leaves a factor of ten; sums in
+    the precision of 16-bit exponent-aligned products would miss it by another ten."""
+    m, rows, k = 3, (512, 512), 2560
+    note("precision", encoding, m, rows, k)
+    raws = [cases.weight(n, k, encoding, 77 + i) for i, n in enumerate(rows)]
+    x = np.random.default_rng(78).standard_normal((m, k)).astype(np.float16)
+    for got, raw, n in zip(run(hip_device, "gguf_gemv_group", x, raws, encoding, rows, count=2), raws, rows):
+        want, _ = reference(x, raw, encoding, n, k)
+        assert np.linalg.norm(got - want) <= 2.0 ** -20 * np.linalg.norm(want), encoding
