@@ -336,8 +336,15 @@ bool gemv_rows_single(const GemvArgs& a) {
 // columns at M = 4: one launch of 3.4 us against three of 2.5 to 2.9).  Matrices that the tuned M =
 // 1 kernels stream faster each by itself keep them from 32 M elements (2 x 12288 x 4096 Q6_K: 18.4
 // against 18.9 us; 6144 x 4096 in three matrices, Q8_0: 12.4 against 8.3).
+// So do wide Q4_K matrices at M > 4, each on the sector kernel (2 x 12288 x 4096 at M = 8 22.5 us in two
+// launches against 26.5; at M = 4 both 18.0).
 bool gemv_rows_group(const GemvArgs* a, int count) {
   if (count < 2 || a[0].x_f32 || a[0].m < 1 || a[0].m > kGemvMaxM || a[0].k > kRowsMaxK) return false;
+  if (a[0].type == kQ4_K && a[0].m > 4 && a[0].k % 1024 == 0) {
+    int narrowest = a[0].n;
+    for (int i = 1; i < count; ++i) narrowest = std::min(narrowest, a[i].n);
+    if (narrowest >= 8192) return false;
+  }
   if (a[0].m > 1 || a[0].k % 2048 != 0) return true;
   int64_t elements = 0;
   for (int i = 0; i < count; ++i) elements += (int64_t)a[i].n * a[i].k;
