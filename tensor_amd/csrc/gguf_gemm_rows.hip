@@ -17,12 +17,13 @@
 // What bounds it: what a CU reads, weights and its workgroup's activations (64 KB a row tile at M = 32
 // and K = 1024) through L2, hence the split of M over workgroups where the matrix is narrow.
 // Microseconds per launch (graph replays, weights rotated), pipelined tiles with their reduce or the
-// per-element small-M kernel -> here: Q4_K gate + up 24576 x 4096 at M = 9 / 32 / 64 41 / 42 / 44 -> 17 / 24
-// / 37; q + k + v 6144 x 4096 at M = 32 Q4_K 23.5 -> 11.8, Q6_K 40.3 -> 15.1; Q6_K 4096 x 12288
-// 36.7 -> 26.3; Q5_0 12288 x 4096 55.5 -> 18.5; packed form, fp32 x, 4096 x 4096 at M = 8 Q3_K 18.1 -> 8.5.
+// per-element small-M kernel -> here: Q4_K gate + up 2 x 12288 x 4096 at M = 9 / 32 / 64 42 / 44 / 46 -> 18 / 26
+// / 39; q + k + v (4096, 1024, 1024) x 4096 at M = 32 Q4_K 18.3 -> 14.0, Q6_K 28.8 -> 16.0; Q6_K 4096 x 12288
+// 36.1 -> 26.5; Q5_0 12288 x 4096 56.7 -> 19.1; packed form, fp32 x, 4096 x 4096 at M = 8 Q3_K 18.1 -> 8.5.
 #include <algorithm>
 
 #include "gguf_rows.h"
+#include "gguf_rows_plan.h"
 
 namespace tensor_gguf {
 namespace {
@@ -35,8 +36,6 @@ struct GemmRowsMore {
   int blocks;                          // workgroups of all matrices, for one set of activation rows
   bool out_half, group;
 };
-
-constexpr int kXRegs = 8;  // 16-byte activation chunks of the next slice a thread holds
 
 // XT = float: fp32 activations (the packed call form), rounded to fp16 as they are staged.
 template <int TYPE, int MT, typename XT>
@@ -243,28 +242,16 @@ template <int TYPE>
 hipError_t launch_rows_type(GemmRowsLaunch& l, hipStream_t stream) {
   using U = Unit<TYPE>;
   const GemmGroupArgs& a = *l.a;
-  int tiles = 0;
-  for (int i = 0; i < a.count; ++i) tiles += (a.n[i] + 15) / 16;
   const int steps = (a.k + 255) / 256;
-  l.waves = 12;
-  // Activation rows per workgroup (16, 32 or 64) and row tiles, for about one workgroup per CU: what a
-  // workgroup reads per 16 columns is 16 per tiles of weights and 16 MT rows of activations.
-  const int m16 = (a.m + 15) / 16;
-  int mt = 0;
-  long best = 0;
-  for (int t : {1, 2, 4}) {
-    const int splits = (m16 + t - 1) / t;
-    const int per = std::min(12, (tiles * splits + 255) / 256);
-    const long rounds = ((long)(tiles + per - 1) / per * splits + 255) / 256;
-    const long cost = rounds * (16L * per * Block<TYPE>::BYTES / Block<TYPE>::QK + 32L * t);
-    if (mt == 0 || cost < best) mt = t, best = cost;
-  }
-  l.m_splits = (m16 + mt - 1) / mt;
-  l.per = std::min(12, (tiles * l.m_splits + 255) / 256);
-  const int m = std::min(a.m, 16 * mt);
+  l.waves = kRowsWaves;
+  const GemmRowsPlan plan = plan_gemm_rows(a.n, a.count, a.m, a.k, (double)Block<TYPE>::BYTES / Block<TYPE>::QK,
+                                           a.x_f32);
+  l.m_splits = plan.m_splits;
+  l.per = plan.per;
+  const int m = std::min(a.m, 16 * plan.t);
   // the slice that the threads' registers and LDS hold
   const int lds_x = 158 * 1024 - l.waves * 16 * U::ROW - 16 * m;
-  l.slice_steps = std::min({steps, kXRegs * l.waves * 64 * 16 / (m * (a.x_f32 ? 1024 : 512)), lds_x / (m * 512)});
+  l.slice_steps = std::min({steps, gemm_rows_slice(m, a.x_f32), lds_x / (m * 512)});
   if (l.slice_steps < 1) return hipErrorInvalidValue;
   l.split = std::max(1, std::min(l.waves / l.per, l.slice_steps));
   if (l.slice_steps < steps) l.slice_steps = l.slice_steps / l.split * l.split;  // every wave a whole share
@@ -278,7 +265,7 @@ hipError_t launch_rows_type(GemmRowsLaunch& l, hipStream_t stream) {
   if (l.m_splits > 1) l.grid = (l.grid + 7) / 8 * 8 * l.m_splits;
   l.lds = std::max((size_t)m * (l.slice_steps * 512 + 16) + (size_t)l.waves * 16 * U::ROW,
                    (size_t)l.per * l.split * m * 64);
-  switch (mt) {
+  switch (plan.t) {
     case 1: return launch_rows<TYPE, 1>(l, stream);
     case 2: return launch_rows<TYPE, 2>(l, stream);
     default: return launch_rows<TYPE, 4>(l, stream);

@@ -1,0 +1,67 @@
+// Launch shapes of the kernels that stream 16-row tiles (gguf_gemm_rows.hip): plain host code without HIP,
+// so that a CPU test can compile it by itself.
+#pragma once
+
+#include <algorithm>
+
+namespace tensor_gguf {
+
+// The streaming GEMM's launch: workgroups of `per` row tiles and 16 t activation rows, m_splits of
+// which share a set of weight rows.
+struct GemmRowsPlan {
+  int t, per, m_splits;
+};
+
+constexpr int kRowsWaves = 12;  // waves of a streaming GEMM workgroup, one workgroup a CU
+
+// Workgroups of one set of activation rows: row tiles are grouped within a matrix, so each
+// matrix rounds up by itself.
+inline long rows_blocks(const int* n, int count, int per) {
+  long blocks = 0;
+  for (int i = 0; i < count; ++i) blocks += ((n[i] + 15) / 16 + per - 1) / per;
+  return blocks;
+}
+
+// Rounds of the 256 CUs that a launch takes: the sets of weight rows go round the eight XCDs in turn,
+// each with its m_splits workgroups (32 CUs an XCD).
+inline long gemm_rows_rounds(const int* n, int count, const GemmRowsPlan& plan) {
+  return ((rows_blocks(n, count, plan.per) + 7) / 8 * plan.m_splits + 31) / 32;
+}
+
+// 256-column steps of an activation slice of `rows` rows that a workgroup's threads hold in registers.
+constexpr int kXRegs = 8;  // 16-byte activation chunks of the next slice a thread holds
+inline int gemm_rows_slice(int rows, bool x_f32) {
+  return kXRegs * kRowsWaves * 64 * 16 / (rows * (x_f32 ? 1024 : 512));
+}
+
+// The (t, per) of least cost, rounds x what a workgroup takes: its start and end, and for each 256
+// columns the decode, products and weights of its tiles (over fewer waves where a slice has fewer steps
+// than a tile has waves) and the staging of its activations.  In units of ~15 ns, fitted to
+// 420 shapes and row counts of Q4_K, Q6_K, Q8_0, Q5_0 and Q2_K timed at every (t, per): the choice is 0.7%
+// slower than the best on average, 11% at the 99th percentile.  Counting tiles over all matrices
+// instead of the workgroups launched, and reads without the decode, took a second round for four workgroups or
+// decoded everything four times: q + k + v (4096, 1024, 1024) x 4096 Q4_K at M = 32 23.5 -> 14.0 us, at M =
+// 64 34.9 -> 18.2; 3 x 4096 rows at M = 32 36.0 -> 19.0; 8192 columns, (8192, 1024, 1024), Q8_0 at M =
+// 48 83.8 -> 42.9.
+inline GemmRowsPlan plan_gemm_rows(const int* n, int count, int m, int k, double bytes_per_element, bool x_f32) {
+  const int m16 = (m + 15) / 16, steps = (k + 255) / 256;
+  GemmRowsPlan best{1, 1, m16};
+  double least = 0;
+  for (int t : {1, 2, 4}) {
+    if (t > 1 && t >= 2 * m16) break;  // no more rows than M
+    const int rows = std::min(m, 16 * t), slice = std::max(1, gemm_rows_slice(rows, x_f32));
+    const double staging = rows * (rows > 48 && steps > slice ? 1.6 : 1.0);
+    for (int per = 1; per <= kRowsWaves; ++per) {
+      const GemmRowsPlan plan{t, per, (m16 + t - 1) / t};
+      const long rounds = gemm_rows_rounds(n, count, plan);
+      const int waves = kRowsWaves / per;  // of a tile
+      const double idle = steps > slice && slice < waves ? (double)waves / slice : 1.0;
+      const double cost = rounds * (150 + steps * (per * (7 + 2 * t + 7 * bytes_per_element) * idle + staging));
+      if (least == 0 || cost < least) best = plan, least = cost;
+      if (rounds == 1) break;  // more tiles only make that round longer
+    }
+  }
+  return best;
+}
+
+}  // namespace tensor_gguf

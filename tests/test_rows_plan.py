@@ -1,0 +1,71 @@
+"""Launch shapes of the 16-row-tile kernels (csrc/gguf_rows_plan.h), compiled as plain host code (CPU only)."""
+
+from __future__ import annotations
+
+import ctypes as c
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from tensor_amd.gguf import quant as Q
+
+CSRC = Path(__file__).resolve().parents[1] / "tensor_amd" / "csrc"
+SOURCE = """
+#include "gguf_rows_plan.h"
+using namespace tensor_gguf;
+extern "C" void gemm_rows(const int* n, int count, int m, int k, double bytes, int* out) {
+  const GemmRowsPlan p = plan_gemm_rows(n, count, m, k, bytes, false);
+  out[0] = p.t, out[1] = p.per, out[2] = p.m_splits;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("rows_plan")
+    (folder / "plan.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", str(CSRC),
+                    str(folder / "plan.cpp"), "-o", str(folder / "plan.so")], check=True, capture_output=True)
+    return c.CDLL(str(folder / "plan.so"))
+
+
+def blocks(rows, per):
+    return sum(-(-(-(-n // 16)) // per) for n in rows)
+
+
+def gemm_rows(library, encoding, m, k, rows):
+    qk, size = Q.GEOMETRY[Q.ggml_type(encoding)]
+    out = (c.c_int * 3)()
+    library.gemm_rows((c.c_int * len(rows))(*rows), len(rows), m, k, c.c_double(size / qk), out)
+    return tuple(out)
+
+
+@pytest.mark.parametrize("encoding", ["q2_k", "q4_k", "q6_k", "q8_0"])
+@pytest.mark.parametrize("rows,k", [((4096, 1024, 1024), 4096), ((4096, 4096, 4096), 4096), ((2048, 2048, 2048), 2048),
+                                    ((8192, 1024, 1024), 8192), ((2560, 640, 640), 2560), ((12288, 12288), 4096),
+                                    ((1, 17, 33), 256), ((64000,), 4096)])
+def test_streaming_gemm_counts_the_workgroups_it_launches(library, encoding, rows, k):
+    """Workgroups round up per matrix; no (t, per) that the plan could take has fewer rounds with as little
+    work in each (an extra round for a few workgroups costs as much as a full one)."""
+    def rounds(t, per, m_splits):  # of an XCD's 32 CUs: it takes every eighth set of weight rows
+        return -(-(-(-blocks(rows, per) // 8) * m_splits) // 32)
+
+    for m in (9, 16, 17, 32, 33, 48, 64):
+        t, per, m_splits = gemm_rows(library, encoding, m, k, rows)
+        m16 = -(-m // 16)
+        assert t in (1, 2, 4) and 1 <= per <= 12 and m_splits == -(-m16 // t)
+        assert t == 1 or t < 2 * m16  # no more activation rows than M has
+        mine = rounds(t, per, m_splits)
+        for other_t in (1, 2, 4):
+            for other in range(1, per + 1):
+                splits = -(-m16 // other_t)
+                if other_t <= t and (other_t, other) != (t, per):
+                    assert rounds(other_t, other, splits) > mine, (m, (t, per), (other_t, other))
+
+
+def test_streaming_gemm_keeps_ordinary_groups_in_one_round(library):
+    for m, rows in ((32, (4096, 1024, 1024)), (64, (4096, 1024, 1024)), (32, (4096, 4096, 4096)),
+                    (32, (2048, 2048, 2048)), (48, (2560, 640, 640))):
+        t, per, m_splits = gemm_rows(library, "q4_k", m, 4096, rows)
+        assert -(-blocks(rows, per) // 8) * m_splits <= 32, (m, rows, t, per)
