@@ -39,6 +39,7 @@
 #include <algorithm>
 
 #include "gguf_rows.h"
+#include "gguf_rows_plan.h"
 
 namespace tensor_gguf {
 namespace {
@@ -273,16 +274,10 @@ hipError_t launch_rows_type(RowsLaunch& l, int count, hipStream_t stream) {
   using U = Unit<TYPE>;
   const int m = l.g[0].m, k = l.g[0].k;
   const int pair = l.flags & kRowsSwiglu ? 2 : 1;  // tiles that stay together
-  int tiles = 0;
-  for (int i = 0; i < count; ++i) tiles += (l.g[i].n + 15) / 16;
+  int rows[kGemvGroupMax];
+  for (int i = 0; i < count; ++i) rows[i] = l.g[i].n;
   const int steps = (k + 4 * U::ELEMS - 1) / (4 * U::ELEMS);
-  // Tiles (or pairs) per workgroup, and its waves.  Up to 1024 tiles one workgroup per CU holds them
-  // all and 12 waves (the most that leave a lane 168 registers) share their steps: 12288 x 4096 at M =
-  // 4 (768 tiles) Q4_0 9.4 us with three tiles against 10.0 with one tile and 8 waves.  Larger matrices
-  // go in workgroups of four tiles and 8 waves, two of which fit a CU beside the activations of four
-  // rows: 64000 x 4096 Q6_K at M = 4 45.6 us against 53.0 with 12 waves and 58.6 with one tile.
-  const int groups = std::max(1, std::min(tiles <= 1024 ? (tiles + 255) / 256 : 4, 12 / pair));
-  const int max_waves = tiles <= 1024 ? 12 : 8;
+  const auto [groups, max_waves] = plan_gemv_rows(rows, count, pair > 1);
   l.per = groups * pair;
   const int most = std::max(1, std::min(max_waves / l.per, steps)), rounds = (steps + most - 1) / most;
   l.split = (steps + rounds - 1) / rounds;  // the fewest ranges of that many steps

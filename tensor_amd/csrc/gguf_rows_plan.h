@@ -64,4 +64,25 @@ inline GemmRowsPlan plan_gemm_rows(const int* n, int count, int m, int k, double
   return best;
 }
 
+// The decode GEMV's workgroups: `groups` row tiles (or gate / up tile pairs) of one matrix and at most
+// `waves` waves.
+struct GemvRowsPlan {
+  int groups, waves;
+};
+
+// One workgroup per CU where that holds all tiles, its 12 waves (the most that leave a lane 168
+// registers) sharing their steps: 12288 x 4096 at M = 4 (768 tiles) Q4_0 9.4 us with three tiles against
+// 10.0 with one tile and 8 waves.  The workgroups that are launched count, each matrix rounding up by
+// itself: 3 x 4096 rows of 4096 columns take 258 of three tiles, so four tiles each: Q4_K at M = 4 / 8 17.4 /
+// 22.2 -> 11.7 / 15.0 us, Q8_0 19.7 / 23.3 -> 13.9 / 15.7.  Up to six tiles (2 x 12288 rows, 20000
+// rows: Q4_K at M = 2 / 8 16.7 / 28.0 -> 14.9 / 20.7 and 16.5 / 27.0 -> 14.2 / 18.8).  Larger matrices go in
+// workgroups of four tiles and 8 waves, two of which fit a CU beside the activations of four rows:
+// 64000 x 4096 Q6_K at M = 4 45.6 us against 53.0 with 12 waves and 58.6 with one tile; 2 x 14336 rows
+// Q4_K at M = 2 17.2 us against 18.6 with seven tiles.
+inline GemvRowsPlan plan_gemv_rows(const int* n, int count, bool pair) {
+  for (int groups = 1; groups <= (pair ? 4 : 6); ++groups)
+    if (rows_blocks(n, count, groups) <= 256) return {groups, 12};
+  return {4, 8};
+}
+
 }  // namespace tensor_gguf

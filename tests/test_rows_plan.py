@@ -18,6 +18,10 @@ extern "C" void gemm_rows(const int* n, int count, int m, int k, double bytes, i
   const GemmRowsPlan p = plan_gemm_rows(n, count, m, k, bytes, false);
   out[0] = p.t, out[1] = p.per, out[2] = p.m_splits;
 }
+extern "C" void gemv_rows(const int* n, int count, int pair, int* out) {
+  const GemvRowsPlan p = plan_gemv_rows(n, count, pair);
+  out[0] = p.groups, out[1] = p.waves;
+}
 """
 
 
@@ -69,3 +73,26 @@ def test_streaming_gemm_keeps_ordinary_groups_in_one_round(library):
                     (32, (2048, 2048, 2048)), (48, (2560, 640, 640))):
         t, per, m_splits = gemm_rows(library, "q4_k", m, 4096, rows)
         assert -(-blocks(rows, per) // 8) * m_splits <= 32, (m, rows, t, per)
+
+
+def test_decode_gemv_takes_one_round_of_the_workgroups_it_launches(library):
+    """Up to six row tiles a workgroup (four gate / up pairs), the fewest that leave at most 256
+    workgroups; beyond, workgroups of four and 8 waves."""
+    def plan(rows, pair=False):
+        out = (c.c_int * 2)()
+        library.gemv_rows((c.c_int * len(rows))(*rows), len(rows), int(pair), out)
+        return tuple(out)
+
+    assert plan((4096, 4096, 4096)) == (4, 12)  # three tiles each would be 258 workgroups
+    assert plan((4096, 1024, 1024)) == (2, 12)
+    assert plan((12288, 12288)) == (6, 12)
+    assert plan((14336, 14336)) == (4, 8)
+    for rows in ((1,), (4096,), (4097,), (12288,), (4096, 1024, 1024), (4100, 4100), (5120, 5120, 5120), (64000,),
+                 (24576,), (24577,)):
+        for pair in (False, True):
+            if pair and len(rows) > 1:
+                continue
+            groups, waves = plan(rows, pair)
+            fits = [g for g in range(1, 5 if pair else 7) if blocks(rows, g) <= 256]
+            assert (groups, waves) == ((fits[0], 12) if fits else (4, 8)), (rows, pair)
+            assert groups * (2 if pair else 1) <= waves
