@@ -39,13 +39,14 @@ struct GemmRowsMore {
 
 // XT = float: fp32 activations (the packed call form), rounded to fp16 as they are staged.
 template <int TYPE, int MT, typename XT>
-__global__ __launch_bounds__(768) void gemm_rows(const XT* __restrict__ x, const uint8_t* __restrict__ w0, int n0,
+__global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows(const XT* __restrict__ x, const uint8_t* __restrict__ w0, int n0,
                                                  int k, int m_all, int per, int split, int slice_steps, int m_splits,
                                                  const GemmRowsMore more) {
   using U = Unit<TYPE>;
   constexpr int CHUNKS = U::ELEMS / 8, PER_SUB = U::SUB / 8, SUBS = U::ELEMS / U::SUB;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  const int tid = threadIdx.x, lane = tid & 63, threads = blockDim.x;
+  constexpr int threads = 64 * kRowsWaves;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int wave = scalar(tid >> 6);
   const int col = lane & 15, g = lane >> 4;
 
@@ -219,7 +220,7 @@ __global__ __launch_bounds__(768) void gemm_rows(const XT* __restrict__ x, const
 struct GemmRowsLaunch {
   const GemmGroupArgs* a;
   GemmRowsMore more;
-  int per, split, slice_steps, waves, m_splits, grid;
+  int per, split, slice_steps, m_splits, grid;
   size_t lds;
 };
 
@@ -228,11 +229,11 @@ hipError_t launch_rows(const GemmRowsLaunch& l, hipStream_t stream) {
   const GemmGroupArgs& a = *l.a;
   const uint8_t* w = static_cast<const uint8_t*>(a.w[0]);
   if (a.x_f32)
-    hipLaunchKernelGGL((gemm_rows<TYPE, MT, float>), dim3(l.grid), dim3(64 * l.waves), l.lds, stream,
+    hipLaunchKernelGGL((gemm_rows<TYPE, MT, float>), dim3(l.grid), dim3(64 * kRowsWaves), l.lds, stream,
                        static_cast<const float*>(a.x), w, a.n[0], a.k, a.m, l.per, l.split, l.slice_steps, l.m_splits,
                        l.more);
   else
-    hipLaunchKernelGGL((gemm_rows<TYPE, MT, _Float16>), dim3(l.grid), dim3(64 * l.waves), l.lds, stream,
+    hipLaunchKernelGGL((gemm_rows<TYPE, MT, _Float16>), dim3(l.grid), dim3(64 * kRowsWaves), l.lds, stream,
                        static_cast<const _Float16*>(a.x), w, a.n[0], a.k, a.m, l.per, l.split, l.slice_steps,
                        l.m_splits, l.more);
   return hipGetLastError();
@@ -243,17 +244,16 @@ hipError_t launch_rows_type(GemmRowsLaunch& l, hipStream_t stream) {
   using U = Unit<TYPE>;
   const GemmGroupArgs& a = *l.a;
   const int steps = (a.k + 255) / 256;
-  l.waves = kRowsWaves;
   const GemmRowsPlan plan = plan_gemm_rows(a.n, a.count, a.m, a.k, (double)Block<TYPE>::BYTES / Block<TYPE>::QK,
                                            a.x_f32);
   l.m_splits = plan.m_splits;
   l.per = plan.per;
   const int m = std::min(a.m, 16 * plan.t);
   // the slice that the threads' registers and LDS hold
-  const int lds_x = 158 * 1024 - l.waves * 16 * U::ROW - 16 * m;
+  const int lds_x = 158 * 1024 - kRowsWaves * 16 * U::ROW - 16 * m;
   l.slice_steps = std::min({steps, gemm_rows_slice(m, a.x_f32), lds_x / (m * 512)});
   if (l.slice_steps < 1) return hipErrorInvalidValue;
-  l.split = std::max(1, std::min(l.waves / l.per, l.slice_steps));
+  l.split = std::max(1, std::min(kRowsWaves / l.per, l.slice_steps));
   if (l.slice_steps < steps) l.slice_steps = l.slice_steps / l.split * l.split;  // every wave a whole share
   l.grid = 0;
   for (int i = 0; i < a.count; ++i) {
@@ -263,7 +263,7 @@ hipError_t launch_rows_type(GemmRowsLaunch& l, hipStream_t stream) {
   for (int i = a.count; i < kGemmGroupMax - 1; ++i) l.more.first_block[i] = 0x7fffffff;
   l.more.blocks = l.grid;
   if (l.m_splits > 1) l.grid = (l.grid + 7) / 8 * 8 * l.m_splits;
-  l.lds = std::max((size_t)m * (l.slice_steps * 512 + 16) + (size_t)l.waves * 16 * U::ROW,
+  l.lds = std::max((size_t)m * (l.slice_steps * 512 + 16) + (size_t)kRowsWaves * 16 * U::ROW,
                    (size_t)l.per * l.split * m * 64);
   switch (plan.t) {
     case 1: return launch_rows<TYPE, 1>(l, stream);

@@ -46,7 +46,7 @@ def kernels():
 def test_library_carries_the_hot_path_kernels(kernels):
     names = {k[".name"] for k in kernels}
     for stem in ("gemv_q4k_m1", "gemv_q4k_sec", "gemv_q6k_lds", "gemv_q32_m1", "gemm_pipe", "gemm_reduce",
-                 "gemm_skinny", "dequant_kernel"):
+                 "gemm_skinny", "dequant_kernel", "gemv_rows", "gemm_rows"):
         assert any(stem in name for name in names), stem
 
 
@@ -72,3 +72,19 @@ def test_every_kernel_fits_gfx950(kernels):
         if problems:
             bad.append((name, problems))
     assert not bad, bad[:10]
+
+
+def test_row_tile_kernels_take_few_arguments(kernels):
+    """No hidden arguments (256 bytes a launch, which a kernel that reads blockDim gets), and in the decode GEMV
+    everything but a group's further matrices within the 64 bytes that arrive in registers."""
+    seen = 0
+    for k in kernels:
+        if not any(stem in k[".name"] for stem in ("gemv_rows", "gemm_rows")):
+            continue
+        seen += 1
+        args = k[".args"]
+        assert not [a for a in args if a[".value_kind"].startswith("hidden")], k[".name"]
+        if "gemv_rows" in k[".name"]:
+            assert [a[".value_kind"] for a in args[:3]] == ["global_buffer"] * 3  # x, weights, output
+            assert all(a[".offset"] + a[".size"] <= 64 for a in args[:-1]), k[".name"]
+    assert seen >= 40
