@@ -38,6 +38,7 @@
 // without activations masked off instead of reading zeros (1-3% slower).
 #include <algorithm>
 
+#include "gguf_decode.h"
 #include "gguf_rows.h"
 #include "gguf_rows_plan.h"
 
@@ -66,6 +67,35 @@ __device__ __forceinline__ float sum_pieces(float v) {
   const auto halves = __builtin_amdgcn_permlane32_swap(b, b, false, false);
   const uint32_t h0 = halves[0], h1 = halves[1];
   return __builtin_bit_cast(float, h0) + __builtin_bit_cast(float, h1);
+}
+
+__device__ __forceinline__ bool is_finite(float v) {
+  return (__builtin_bit_cast(uint32_t, v) & 0x7F800000u) != 0x7F800000u;
+}
+
+// A sum that is not finite: an infinity in x makes scale * (codes . x) + low * sum(x) infinity minus
+// infinity, and one in a scale multiplies a sum of either sign, where x . W is defined by each
+// element's product.  The encodings without a vector kernel that sums scale by scale (gemv_blocks
+// multiplies elements) take such outputs again, element by element, a wave to an output: one
+// infinite row of eight at 12288 x 4096 Q5_K 12.5 -> 109 us; the test of each sum costs finite calls 0 to 1%.
+template <int TYPE>
+constexpr bool by_element() {
+  return TYPE == kQ4_1 || TYPE == kQ5_0 || TYPE == kQ5_1 || TYPE == kQ2_K || TYPE == kQ3_K || TYPE == kQ5_K;
+}
+
+// x . (one row of W) over the wave, in every lane.
+template <int TYPE>
+__device__ __forceinline__ float element_product(const uint8_t* __restrict__ row, const _Float16* __restrict__ x, int k, int lane) {
+  float sum = 0.0f;
+#pragma unroll 1
+  for (int e = 8 * lane; e < k; e += 512) {
+    float v[8];
+    decode8<TYPE>(row + (size_t)(e / Block<TYPE>::QK) * Block<TYPE>::BYTES, e % Block<TYPE>::QK, v);
+    const half8_t xv = *reinterpret_cast<const half8_t*>(x + e);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sum = fmaf(v[i], (float)xv[i], sum);
+  }
+  return wave_sum(sum);
 }
 
 constexpr int kRowsZero = 256;  // bytes of zeros in LDS that inactive lanes read
@@ -233,10 +263,12 @@ __global__ __launch_bounds__(768) void gemv_rows(const _Float16* __restrict__ x,
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   const int step = pair ? 2 : 1, outputs = (pair ? per >> 1 : per) * tile_items;
   const float inv_items = inverse(tile_items);
-  for (int o = tid; o < outputs; o += threads) {
-    const int t = quotient(o, inv_items), in_tile = o - t * tile_items;
+  for (int first = 64 * wave; first < outputs; first += threads) {
+    const int o = min(first + lane, outputs - 1);
+    const int t = quotient(o, inv_items), in_tile = o - t * tile_items, m = in_tile >> 4;
     const float* p = partial + t * step * split * tile_items + in_tile;
     const int row = (tile_of_block + t) * 16 + (in_tile & 15);
+    const bool live = first + lane < outputs && row < n;
     auto over_ranges = [&](const float* from) {  // in range order, four reads in flight
       float v = 0.0f;
       for (int q = 0; q < split; q += 4) {
@@ -248,10 +280,21 @@ __global__ __launch_bounds__(768) void gemv_rows(const _Float16* __restrict__ x,
       }
       return v;
     };
-    float v = over_ranges(p);
-    if (pair) v = swiglu(v, over_ranges(p + split * tile_items));
-    if (row >= n) continue;
-    const size_t index = (size_t)(in_tile >> 4) * n + row;
+    float v = over_ranges(p), up = 0.0f;
+    if (pair) up = over_ranges(p + split * tile_items);
+    if constexpr (by_element<TYPE>()) {
+      for (uint64_t rest = __builtin_amdgcn_ballot_w64(live && !(is_finite(v) && is_finite(up))); rest; rest &= rest - 1) {
+        const int l = __builtin_ctzll(rest);
+        const size_t at = (size_t)__builtin_amdgcn_readlane(row, l) * (size_t)(blocks * Block<TYPE>::BYTES);
+        const _Float16* xm = x + (size_t)__builtin_amdgcn_readlane(m, l) * k;
+        const float exact = element_product<TYPE>(w + at, xm, k, lane);
+        const float exact_up = pair ? element_product<TYPE>(more.w[0] + at, xm, k, lane) : 0.0f;
+        if (lane == l) v = exact, up = exact_up;
+      }
+    }
+    if (pair) v = swiglu(v, up);
+    if (!live) continue;
+    const size_t index = (size_t)m * n + row;
     if (flags & kRowsHalf) store_out(static_cast<_Float16*>(out), index, v);
     else store_out(static_cast<float*>(out), index, v);
   }

@@ -130,3 +130,52 @@ def test_sums_keep_fp32_precision(hip_device, encoding):
     for got, raw, n in zip(run(hip_device, "gguf_gemv_group", x, raws, encoding, rows, count=2), raws, rows):
         want, _ = reference(x, raw, encoding, n, k)
         assert np.linalg.norm(got - want) <= 2.0 ** -20 * np.linalg.norm(want), encoding
+
+
+def by_elements(x, w):
+    """x W^T element by element: what an infinity or a NaN in either makes of each output."""
+    with np.errstate(all="ignore"):
+        return np.stack([(row.astype(np.float64) * w.astype(np.float64)).sum(1) for row in x])
+
+
+def same_kind(got, want):
+    return (np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+            and np.array_equal(np.isneginf(got), np.isneginf(want)))
+
+
+@pytest.mark.parametrize("encoding", ["q4_1", "q5_0", "q5_1", "q2_k", "q3_k", "q5_k"])
+@pytest.mark.parametrize("m", [1, 3, 8])
+def test_infinities_and_nans_are_those_of_the_elements_products(hip_device, encoding, m):
+    """An infinite activation gives infinities of the weights' signs (NaN at a zero weight, and for two that
+    disagree), an infinite scale what its elements' products sum to; other rows stay as they are."""
+    k, rows = 2592 if Q.GEOMETRY[Q.ggml_type(encoding)][0] == 32 else 2304, (200, 33)
+    note("infinities", encoding, m, rows, k)
+    raws = [cases.weight(n, k, encoding, 61 + i) for i, n in enumerate(rows)]
+    size = Q.GEOMETRY[Q.ggml_type(encoding)][1]
+    offset = cases.HALF_FIELDS[Q.ggml_type(encoding)][0]
+    raws[1] = raws[1].copy()
+    raws[1][5, 3 * size + offset:3 * size + offset + 2] = np.array([np.inf], np.float16).view(np.uint8)
+    raws[1][32, offset:offset + 2] = np.array([np.nan], np.float16).view(np.uint8)
+    with np.errstate(all="ignore"):
+        weights = [R.dequantize(raw, Q.ggml_type(encoding), n, k) for raw, n in zip(raws, rows)]
+    for special in ((np.inf,), (-np.inf,), (np.inf, np.inf), (np.nan,), ()):
+        x = cases.activation(m, k, 63)
+        for i, value in enumerate(special):
+            x[0, 700 + 800 * i] = value
+        group = run(hip_device, "gguf_gemv_group", x, raws, encoding, rows, count=2)
+        for got, w, n in zip(group, weights, rows):
+            want = by_elements(x, w)
+            assert same_kind(got, want), (encoding, m, n, special)
+            finite = np.isfinite(want)
+            with np.errstate(all="ignore"):
+                bound = k * 2.0 ** -24 * 3 * np.abs(x.astype(np.float64)).sum(1)[:, None] * np.abs(w).max(1)[None, :] + 1e-12
+            assert (np.abs(got[finite] - want[finite]) <= bound[finite]).all()
+    # the SwiGLU pair takes its own two sums
+    gate, up = cases.weight(4130, k, encoding, 65), cases.weight(4130, k, encoding, 66)
+    x = cases.activation(m, k, 67)
+    x[0, 700] = np.inf
+    got, = run(hip_device, "gguf_gemv_swiglu", x, [gate, up], encoding, (4130,))
+    g, u = (by_elements(x, R.dequantize(raw, Q.ggml_type(encoding), 4130, k)).astype(np.float32) for raw in (gate, up))
+    with np.errstate(all="ignore"):
+        want = g / (1 + np.exp(-g)) * u
+    assert same_kind(got, want), (encoding, m)
