@@ -77,7 +77,7 @@ __device__ __forceinline__ bool is_finite(float v) {
 // infinity, and one in a scale multiplies a sum of either sign, where x . W is defined by each
 // element's product.  The encodings without a vector kernel that sums scale by scale (gemv_blocks
 // multiplies elements) take such outputs again, element by element, a wave to an output: one
-// infinite row of eight at 12288 x 4096 Q5_K 12.5 -> 109 us; the test of each sum costs finite calls 0 to 1%.
+// infinite row of eight at 12288 x 4096 Q5_K 12.5 -> 109 us; the test of each sum costs finite calls 0 to 2%.
 template <int TYPE>
 constexpr bool by_element() {
   return TYPE == kQ4_1 || TYPE == kQ5_0 || TYPE == kQ5_1 || TYPE == kQ2_K || TYPE == kQ3_K || TYPE == kQ5_K;
@@ -283,7 +283,8 @@ __global__ __launch_bounds__(768) void gemv_rows(const _Float16* __restrict__ x,
     float v = over_ranges(p), up = 0.0f;
     if (pair) up = over_ranges(p + split * tile_items);
     if constexpr (by_element<TYPE>()) {
-      for (uint64_t rest = __builtin_amdgcn_ballot_w64(live && !(is_finite(v) && is_finite(up))); rest; rest &= rest - 1) {
+      uint64_t rest = __builtin_amdgcn_ballot_w64(live && !(is_finite(v) && is_finite(up)));
+      for (; __builtin_expect(rest != 0, 0); rest &= rest - 1) {
         const int l = __builtin_ctzll(rest);
         const size_t at = (size_t)__builtin_amdgcn_readlane(row, l) * (size_t)(blocks * Block<TYPE>::BYTES);
         const _Float16* xm = x + (size_t)__builtin_amdgcn_readlane(m, l) * k;
@@ -324,7 +325,7 @@ hipError_t launch_rows_type(RowsLaunch& l, int count, hipStream_t stream) {
   int rows[kGemvGroupMax];
   for (int i = 0; i < count; ++i) rows[i] = l.g[i].n;
   const int steps = (k + 4 * U::ELEMS - 1) / (4 * U::ELEMS);
-  const auto [groups, max_waves] = plan_gemv_rows(rows, count, pair > 1);
+  const auto [groups, max_waves] = plan_gemv_rows(rows, count, m, pair > 1);
   l.per = groups * pair;
   const int most = std::max(1, std::min(max_waves / l.per, steps)), rounds = (steps + most - 1) / most;
   l.split = (steps + rounds - 1) / rounds;  // the fewest ranges of that many steps
@@ -374,23 +375,11 @@ bool gemv_rows_single(const GemvArgs& a) {
   }
 }
 
-// A group in one launch saves a launch per further matrix (q, k, v of 1024 + 2 x 128 rows and 1024
-// columns at M = 4: one launch of 3.4 us against three of 2.5 to 2.9).  Matrices that the tuned M =
-// 1 kernels stream faster each by itself keep them from 32 M elements (2 x 12288 x 4096 Q6_K: 18.4
-// against 18.9 us; 6144 x 4096 in three matrices, Q8_0: 12.4 against 8.3).
-// So do wide Q4_K matrices at M > 4, each on the sector kernel (2 x 12288 x 4096 at M = 8 22.5 us in two
-// launches against 26.5; at M = 4 both 18.0).
 bool gemv_rows_group(const GemvArgs* a, int count) {
   if (count < 2 || a[0].x_f32 || a[0].m < 1 || a[0].m > kGemvMaxM || a[0].k > kRowsMaxK) return false;
-  if (a[0].type == kQ4_K && a[0].m > 4 && a[0].k % 1024 == 0) {
-    int narrowest = a[0].n;
-    for (int i = 1; i < count; ++i) narrowest = std::min(narrowest, a[i].n);
-    if (narrowest >= 8192) return false;
-  }
-  if (a[0].m > 1 || a[0].k % 2048 != 0) return true;
-  int64_t elements = 0;
-  for (int i = 0; i < count; ++i) elements += (int64_t)a[i].n * a[i].k;
-  return elements < (int64_t)32 << 20;
+  int rows[kGemvGroupMax];
+  for (int i = 0; i < count; ++i) rows[i] = a[i].n;
+  return gemv_rows_group_better(rows, count, a[0].m, a[0].k);
 }
 
 // SwiGLU pairs: as single matrices, with the lines where the vector pair kernels (one wave per output row)

@@ -264,7 +264,5 @@ __device__ __forceinline__ float inverse(int b) { return __builtin_amdgcn_rcpf((
 __device__ __forceinline__ int quotient(int a, float inv) { return (int)(((float)a + 0.5f) * inv); }
 __device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-constexpr int kRowsMaxK = 1 << 22;  // 16 rows stay within the 32-bit offsets of a tile
-
 }  // namespace
 }  // namespace tensor_gguf

@@ -1,10 +1,15 @@
-// Launch shapes of the kernels that stream 16-row tiles (gguf_gemm_rows.hip): plain host code without HIP,
-// so that a CPU test can compile it by itself.
+// Launch shapes of the kernels that stream 16-row tiles (gguf_gemv_rows.hip, gguf_gemm_rows.hip), and the
+// lines between them and the kernels they stand beside: plain host code without HIP, so that a CPU
+// test can compile it by itself.
 #pragma once
 
 #include <algorithm>
 
+#include "gguf_types.h"
+
 namespace tensor_gguf {
+
+constexpr int kRowsMaxK = 1 << 22;  // 16 rows stay within the 32-bit offsets of a tile
 
 // The streaming GEMM's launch: workgroups of `per` row tiles and 16 t activation rows, m_splits of
 // which share a set of weight rows.
@@ -75,14 +80,27 @@ struct GemvRowsPlan {
 // 10.0 with one tile and 8 waves.  The workgroups that are launched count, each matrix rounding up by
 // itself: 3 x 4096 rows of 4096 columns take 258 of three tiles, so four tiles each: Q4_K at M = 4 / 8 17.4 /
 // 22.2 -> 11.7 / 15.0 us, Q8_0 19.7 / 23.3 -> 13.9 / 15.7.  Up to six tiles (2 x 12288 rows, 20000
-// rows: Q4_K at M = 2 / 8 16.7 / 28.0 -> 14.9 / 20.7 and 16.5 / 27.0 -> 14.2 / 18.8).  Larger matrices go in
-// workgroups of four tiles and 8 waves, two of which fit a CU beside the activations of four rows:
-// 64000 x 4096 Q6_K at M = 4 45.6 us against 53.0 with 12 waves and 58.6 with one tile; 2 x 14336 rows
+// rows: Q4_K at M = 2 / 8 16.7 / 28.0 -> 14.9 / 20.7 and 16.5 / 27.0 -> 14.2 / 18.8), eight where M > 4
+// (2 x 14336 rows Q4_K at M = 6 27.3 -> 22.8, 32000 rows 29.1 -> 24.3).  Larger matrices go in workgroups of four
+// tiles and 8 waves, two of which fit a CU beside the activations of four rows: 64000 x 4096 Q6_K at M = 4 45.6 us against 53.0 with 12 waves and 58.6 with one tile; 2 x 14336 rows
 // Q4_K at M = 2 17.2 us against 18.6 with seven tiles.
-inline GemvRowsPlan plan_gemv_rows(const int* n, int count, bool pair) {
-  for (int groups = 1; groups <= (pair ? 4 : 6); ++groups)
+inline GemvRowsPlan plan_gemv_rows(const int* n, int count, int m, bool pair) {
+  for (int groups = 1; groups <= (pair ? 4 : m > 4 ? 8 : 6); ++groups)
     if (rows_blocks(n, count, groups) <= 256) return {groups, 12};
   return {4, 8};
+}
+
+// Whether a group of two or three matrices goes in one launch, which saves a launch per further matrix (q, k, v
+// of 1024 + 2 x 128 rows and 1024 columns at M = 4: one launch of 3.4 us against three of 2.5 to 2.9).
+// Matrices that the tuned M = 1 kernels stream faster each by itself keep them from 32 M elements (2 x 12288 x
+// 4096 Q6_K: 18.4 against 18.9 us; 6144 x 4096 in three matrices, Q8_0: 12.4 against 8.3).  Wide Q4_K
+// matrices at M > 4 are no exception: with the workgroups of plan_gemv_rows 2 x 12288 rows of 4096 columns take
+// 20.7 us at M = 8 against 22.5 in two launches, 2 x 28672 x 8192 93 against 117, 2 x 12288 x 12288 57 against 90.
+inline bool gemv_rows_group_better(const int* n, int count, int m, int k) {
+  if (m > 1 || k % 2048 != 0) return true;
+  long long elements = 0;
+  for (int i = 0; i < count; ++i) elements += (long long)n[i] * k;
+  return elements < 32ll << 20;
 }
 
 }  // namespace tensor_gguf

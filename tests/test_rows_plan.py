@@ -18,10 +18,11 @@ extern "C" void gemm_rows(const int* n, int count, int m, int k, double bytes, i
   const GemmRowsPlan p = plan_gemm_rows(n, count, m, k, bytes, false);
   out[0] = p.t, out[1] = p.per, out[2] = p.m_splits;
 }
-extern "C" void gemv_rows(const int* n, int count, int pair, int* out) {
-  const GemvRowsPlan p = plan_gemv_rows(n, count, pair);
+extern "C" void gemv_rows(const int* n, int count, int m, int pair, int* out) {
+  const GemvRowsPlan p = plan_gemv_rows(n, count, m, pair);
   out[0] = p.groups, out[1] = p.waves;
 }
+extern "C" int gemv_group(const int* n, int count, int m, int k) { return gemv_rows_group_better(n, count, m, k); }
 """
 
 
@@ -76,23 +77,33 @@ def test_streaming_gemm_keeps_ordinary_groups_in_one_round(library):
 
 
 def test_decode_gemv_takes_one_round_of_the_workgroups_it_launches(library):
-    """Up to six row tiles a workgroup (four gate / up pairs), the fewest that leave at most 256
-    workgroups; beyond, workgroups of four and 8 waves."""
-    def plan(rows, pair=False):
+    """Up to six row tiles a workgroup (eight where M > 4, four gate / up pairs), the fewest that leave at
+    most 256 workgroups; beyond, workgroups of four and 8 waves."""
+    def plan(rows, m=1, pair=False):
         out = (c.c_int * 2)()
-        library.gemv_rows((c.c_int * len(rows))(*rows), len(rows), int(pair), out)
+        library.gemv_rows((c.c_int * len(rows))(*rows), len(rows), m, int(pair), out)
         return tuple(out)
 
     assert plan((4096, 4096, 4096)) == (4, 12)  # three tiles each would be 258 workgroups
     assert plan((4096, 1024, 1024)) == (2, 12)
     assert plan((12288, 12288)) == (6, 12)
-    assert plan((14336, 14336)) == (4, 8)
+    assert plan((14336, 14336), 4) == (4, 8) and plan((14336, 14336), 5) == (7, 12)
     for rows in ((1,), (4096,), (4097,), (12288,), (4096, 1024, 1024), (4100, 4100), (5120, 5120, 5120), (64000,),
-                 (24576,), (24577,)):
-        for pair in (False, True):
+                 (24576,), (24577,), (32768,), (8192, 8192, 8192)):
+        for m, pair in ((1, False), (4, False), (5, False), (8, False), (1, True), (8, True)):
             if pair and len(rows) > 1:
                 continue
-            groups, waves = plan(rows, pair)
-            fits = [g for g in range(1, 5 if pair else 7) if blocks(rows, g) <= 256]
-            assert (groups, waves) == ((fits[0], 12) if fits else (4, 8)), (rows, pair)
+            groups, waves = plan(rows, m, pair)
+            fits = [g for g in range(1, 5 if pair else 9 if m > 4 else 7) if blocks(rows, g) <= 256]
+            assert (groups, waves) == ((fits[0], 12) if fits else (4, 8)), (rows, m, pair)
             assert groups * (2 if pair else 1) <= waves
+
+
+@pytest.mark.parametrize("rows,k", [((12288, 12288), 4096), ((28672, 28672), 7168), ((28672, 28672), 8192),
+                                    ((12288, 12288), 12288), ((8192, 8192), 2048)])
+def test_groups_of_more_rows_than_one_go_in_one_launch(library, rows, k):
+    """Wide ones too, whatever the single-matrix kernels would hold in LDS at that K."""
+    for m in range(2, 9):
+        assert library.gemv_group((c.c_int * len(rows))(*rows), len(rows), m, k)
+    assert not library.gemv_group((c.c_int * len(rows))(*rows), len(rows), 1, k - k % 2048 + 2048)
+    assert library.gemv_group((c.c_int * 3)(1024, 128, 128), 3, 1, 2048)
