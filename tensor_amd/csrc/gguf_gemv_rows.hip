@@ -348,31 +348,9 @@ hipError_t launch_rows_type(RowsLaunch& l, int count, hipStream_t stream) {
 
 }  // namespace
 
-// Matrices of fewer elements than this (in 2^20, by activation rows 1, 2, 3, 4, more) stay on the
-// vector kernels, which reach their result sooner where latency is all: a launch of this kernel takes
-// ~1 us longer before its first product (1024 x 1024 at M = 1: Q4_0 3.0 against 2.3 us).  The lines
-// lie where graph replays of both sides crossed (shapes of 1 to 67 M elements, every encoding).
 bool gemv_rows_single(const GemvArgs& a) {
   if (a.x_f32 || a.m < 1 || a.m > kGemvMaxM || a.k > kRowsMaxK) return false;
-  const int64_t elements = (int64_t)a.n * a.k;
-  const int at = std::min(a.m, 5) - 1;
-  auto from = [&](const int (&millions)[5]) { return elements >= (int64_t)millions[at] << 20; };
-  const bool whole_step = a.m == 1 && a.k % 4096 == 0 && a.k <= 16384;  // row lengths of the tuned M = 1 kernels
-  const bool half_step = a.m == 1 && a.k % 2048 == 0 && a.k <= 16384;
-  switch (a.type) {
-    case kQ4_0: return !half_step && from({32, 16, 3, 3, 2});
-    case kQ4_1: return !half_step && from({16, 16, 16, 6, 6});
-    case kQ5_0: return !half_step && from({16, 6, 6, 3, 6});
-    case kQ5_1: return !half_step && from({16, 16, 16, 6, 6});
-    case kQ8_0: return !half_step && from({16, 16, 6, 3, 2});
-    case kQ2_K: return !whole_step && from({16, 6, 6, 6, 6});
-    case kQ3_K: return !whole_step && from({6, 6, 3, 3, 3});
-    case kQ5_K: return !whole_step && from({6, 6, 3, 2, 2});
-    case kQ6_K: return !(whole_step && a.k <= 12288) && from({16, 2, 3, 2, 3});
-    // M > 1: the plans of tensor_gguf_gemv_plan_v1; M = 1: rows of less than 2048 columns are level
-    case kQ4_K: return a.m == 1 && !whole_step && a.k >= 2048;
-    default: return false;
-  }
+  return gemv_rows_single_better(a.type, a.m, a.n, a.k);
 }
 
 bool gemv_rows_group(const GemvArgs* a, int count) {
@@ -382,16 +360,9 @@ bool gemv_rows_group(const GemvArgs* a, int count) {
   return gemv_rows_group_better(rows, count, a[0].m, a[0].k);
 }
 
-// SwiGLU pairs: as single matrices, with the lines where the vector pair kernels (one wave per output row)
-// crossed: 2 x 3072 x 1024 at M = 2 Q8_0 4.4 against 4.9 us, at M = 4 6.1 against 5.0; 2 x 6912 x
-// 2560 at M = 1 15.4 against 11.3.  Q4_K and Q5_K at M = 1 keep their tuned row lengths; Q4_K at M > 1
-// always comes here (12288 x 4096 at M = 4 about 16 us, 18.5 on the sector kernel in pairs that this replaced).
 bool gemv_rows_pair(const GemvArgs& a) {
   if (a.x_f32 || a.m < 1 || a.m > kGemvMaxM || a.k > kRowsMaxK) return false;
-  const bool slow = a.type == kQ3_K || a.type == kQ5_K || a.type == kQ6_K;  // pairs costly to decode per lane
-  const int millions = a.type == kQ4_K && a.m >= 2 ? 0 : a.m >= 4 || slow ? 4 : a.m == 3 ? 8 : 16;
-  if ((a.type == kQ4_K || a.type == kQ5_K) && a.m == 1 && a.k % 4096 == 0 && a.k <= 16384) return false;
-  return 2 * (int64_t)a.n * a.k >= (int64_t)millions << 20;
+  return gemv_rows_pair_better(a.type, a.m, a.n, a.k);
 }
 
 hipError_t launch_gemv_rows(const GemvArgs* g, int count, const void* w_up, hipStream_t stream) {

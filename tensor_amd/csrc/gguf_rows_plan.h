@@ -90,6 +90,56 @@ inline GemvRowsPlan plan_gemv_rows(const int* n, int count, int m, bool pair) {
   return {4, 8};
 }
 
+// Whether a single matrix goes on this kernel rather than on the vector kernels, which reach their result sooner
+// where latency is all (1024 x 1024 at M = 1: Q4_0 3.0 against 2.3 us).  A line for M = 1, 2, 3, 4, 5 to 6 and
+// 7 to 8, in 2^20 elements times sqrt(n / 4096): few rows leave CUs without a tile, so of two matrices of one size the
+// longer rows gain less (Q4_1 at M = 6: 1024 x 6912 9.5 us against 7.1 on the vector kernel, 4096 x 2048 5.4 against
+// 6.2).  They lie where graph replays of both sides crossed, every encoding at 640 to 12288 rows of 512 to 6912 columns:
+// the choice costs up to 8% over the better one near a line, where lines on elements alone cost up to 34%.
+// A band of row lengths moves a line: up to 2048 columns are one pass of the Q4_0 and Q8_0 vector kernels, of which shorter
+// ones leave lanes idle (Q8_0 at M = 4: 3000 x 1536 4.1 us there, 4.5 here; 3000 x 2560 6.9 and 5.8), Q2_K's
+// gains at up to 1024, and Q6_K's from M = 3 beyond 2048 (1024 x 4096 at M = 3 5.0 there, 5.8 here).
+inline bool gemv_rows_single_better(int type, int m, int n, int k) {
+  const double millions = (double)n * k / (1 << 20), size2 = millions * millions * n / 4096;
+  const int at = m <= 4 ? m - 1 : m <= 6 ? 4 : 5;
+  const auto from = [&](const double (&lines)[6], double band = 1) {
+    return size2 >= lines[at] * band * (lines[at] * band);
+  };
+  const bool whole_step = m == 1 && k % 4096 == 0 && k <= 16384;  // row lengths of the tuned M = 1 kernels
+  const bool half_step = m == 1 && k % 2048 == 0 && k <= 16384;
+  const double one_pass = k <= 1024 || k > 2048 ? 1 : m <= 2 ? 1.8 : 2.2;
+  switch (type) {
+    case kQ4_0: return !half_step && from({28, 16.5, 3.7, 2.5, 1, 0.5}, one_pass);
+    case kQ4_1: return !half_step && from({28, 24, 10, 6, 4, 2});
+    case kQ5_0: return !half_step && from({9, 5, 4, 2, 3.5, 0.75});
+    case kQ5_1: return !half_step && from({24, 10, 9, 6, 4, 3.5});
+    case kQ8_0: return !half_step && from({18, 18, 9, 3.5, 1.5, 0.75}, one_pass);
+    case kQ2_K: return !whole_step && from({18, 5, 5, 2, 3.5, 2}, k <= 1024 ? 2 : 1);
+    case kQ3_K: return !whole_step && from({3.5, 2, 1.5, 1.5, 2, 1.5});
+    case kQ5_K: return !whole_step && from({3, 2, 1.5, 0.75, 0.75, 0.75});
+    case kQ6_K: return !(whole_step && k <= 12288) && from({14, 0.5, 2.5, 0.5, 1.4, 0.5}, m >= 3 && k > 2048 ? 2.5 : 1);
+    // M > 1: the plans of tensor_gguf_gemv_plan_v1.  M = 1: rows of 1024 columns are level, of 1536 and 2048 (one
+    // pass there too) take 10 to 22% longer here, of 2560 to 6912 2 to 14% less.
+    case kQ4_K: return m == 1 && !whole_step && k > 2048;
+    default: return false;
+  }
+}
+
+// The same for SwiGLU pairs, in 2^20 elements of both matrices, where the vector pair kernels (one wave per output row)
+// crossed: 2 x 3072 x 1024 at M = 2 Q8_0 4.4 against 4.9 us, at M = 4 6.1 against 5.0; 2 x 6912 x
+// 2560 at M = 1 15.4 against 11.3.  Where their rows are one pass the line lies half as high again at M = 1 and 4 (M =
+// 1, 2 x 4096 x 2048: Q4_0 4.3 against 4.9, Q4_K 4.7 against 5.2; Q8_0 2 x 2000 x 1056 at M = 4 5.1 against 5.6).
+// Q4_K and Q5_K at M = 1 keep their tuned row lengths; Q4_K at M > 1 always comes here (12288 x 4096 at M = 4 about
+// 16 us, 18.5 on the sector kernel in pairs that this replaced).
+inline bool gemv_rows_pair_better(int type, int m, int n, int k) {
+  if ((type == kQ4_K || type == kQ5_K) && m == 1 && k % 4096 == 0 && k <= 16384) return false;
+  if (type == kQ4_K && m >= 2) return true;
+  const bool slow = type == kQ3_K || type == kQ5_K || type == kQ6_K;  // pairs costly to decode per lane
+  const bool one_pass = (type == kQ4_0 || type == kQ8_0 || type == kQ4_K) && k > 1024 && k <= 2048 && (m == 1 || m == 4);
+  const int millions = m >= 4 || slow ? 4 : m == 3 ? 8 : 16;
+  return 2.0 * n * k >= (double)(millions << 20) * (one_pass ? 1.5 : 1);
+}
+
 // Whether a group of two or three matrices goes in one launch, which saves a launch per further matrix (q, k, v
 // of 1024 + 2 x 128 rows and 1024 columns at M = 4: one launch of 3.4 us against three of 2.5 to 2.9).
 // Matrices that the tuned M = 1 kernels stream faster each by itself keep them from 32 M elements (2 x 12288 x

@@ -92,8 +92,8 @@ def test_launch_shapes(hip_device, encoding, m, rows, k):
         check(got, x, raw, encoding, n, k, (encoding, m, n, k))
 
 
-@pytest.mark.parametrize("encoding,m,n,k", [("q4_0", 5, 2100, 1056), ("q8_0", 8, 2100, 1056), ("q3_k", 3, 1300, 2816),
-                                            ("q6_k", 2, 1030, 2304), ("q5_0", 4, 1030, 3104), ("q4_k", 1, 300, 2304)])
+@pytest.mark.parametrize("encoding,m,n,k", [("q4_0", 5, 4100, 1056), ("q8_0", 8, 4100, 1056), ("q3_k", 3, 1300, 2816),
+                                            ("q6_k", 2, 1030, 2304), ("q5_0", 4, 1530, 3104), ("q4_k", 1, 300, 2304)])
 def test_single_matrices(hip_device, encoding, m, n, k):
     """Sizes above the lines from which a single matrix takes the kernel."""
     note("single", encoding, m, n, k)

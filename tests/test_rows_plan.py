@@ -23,6 +23,8 @@ extern "C" void gemv_rows(const int* n, int count, int m, int pair, int* out) {
   out[0] = p.groups, out[1] = p.waves;
 }
 extern "C" int gemv_group(const int* n, int count, int m, int k) { return gemv_rows_group_better(n, count, m, k); }
+extern "C" int gemv_single(int type, int m, int n, int k) { return gemv_rows_single_better(type, m, n, k); }
+extern "C" int gemv_pair(int type, int m, int n, int k) { return gemv_rows_pair_better(type, m, n, k); }
 """
 
 
@@ -107,3 +109,37 @@ def test_groups_of_more_rows_than_one_go_in_one_launch(library, rows, k):
         assert library.gemv_group((c.c_int * len(rows))(*rows), len(rows), m, k)
     assert not library.gemv_group((c.c_int * len(rows))(*rows), len(rows), 1, k - k % 2048 + 2048)
     assert library.gemv_group((c.c_int * 3)(1024, 128, 128), 3, 1, 2048)
+
+
+@pytest.mark.parametrize("encoding,m,n,k,rows", [
+    ("q4_0", 3, 3000, 1056, False), ("q4_0", 3, 2048, 1536, False), ("q4_0", 3, 6912, 2560, True),
+    ("q8_0", 4, 3000, 1056, False), ("q8_0", 6, 2048, 1056, False), ("q8_0", 8, 12288, 4096, True),
+    ("q4_1", 6, 1024, 6912, False), ("q5_1", 4, 1024, 6912, False), ("q4_1", 6, 4096, 2048, True),
+    ("q2_k", 2, 6912, 1024, False), ("q2_k", 1, 2560, 6912, False), ("q2_k", 2, 6912, 1536, True),
+    ("q6_k", 3, 1024, 4096, False), ("q6_k", 6, 1024, 6912, False), ("q6_k", 3, 4096, 4096, True),
+    ("q4_k", 1, 2560, 2048, False), ("q4_k", 1, 2560, 2560, True), ("q4_0", 2, 4096, 4096, False),
+])
+def test_decode_gemv_leaves_single_matrices_that_the_vector_kernels_do_sooner(library, encoding, m, n, k, rows):
+    """Both kernels timed at each: 1.04 to 1.34 times as long on the one that is not taken."""
+    assert bool(library.gemv_single(Q.ggml_type(encoding), m, n, k)) == rows
+
+
+@pytest.mark.parametrize("encoding", ["q4_0", "q4_k", "q8_0"])
+def test_decode_gemv_lines_follow_size(library, encoding):
+    """More rows of the same length never go back to the vector kernels, nor do pairs of them; the tuned M = 1 row
+    lengths stay there at every size."""
+    type_ = Q.ggml_type(encoding)
+    for take in (library.gemv_single, library.gemv_pair):
+        for m in range(1, 9):
+            for k in (256, 1024, 1536, 2048, 2560, 6912):
+                taken = [bool(take(type_, m, n, k)) for n in (1, 16, 640, 1024, 3000, 4096, 12288, 151936)]
+                assert taken == sorted(taken), (m, k)
+    assert not library.gemv_single(type_, 1, 151936, 4096)
+
+
+def test_swiglu_pairs_of_one_pass_rows_stay_on_the_vector_kernels(library):
+    for encoding, m, n, k, rows in (("q4_0", 1, 4096, 2048, False), ("q4_k", 1, 4096, 2048, False),
+                                    ("q8_0", 4, 2000, 1056, False), ("q8_0", 2, 4096, 2048, True),
+                                    ("q4_0", 1, 6912, 2560, True), ("q4_k", 2, 1, 256, True),
+                                    ("q5_k", 1, 4096, 4096, False)):
+        assert bool(library.gemv_pair(Q.ggml_type(encoding), m, n, k)) == rows, (encoding, m, n, k)
