@@ -214,18 +214,15 @@ static hipError_t launch_tile(const GemvArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The small-M kernel where the streaming kernel (gemm_rows_takes) leaves a call to it or a plan asks: M <= 64
-// for shapes on the generic tiles, and for shapes the pipelined tiles take also N <= 4096.
 bool gemm_small_m(const GemvArgs& a) {
-  if (!gemm_skinny_supported(a)) return false;
-  return !gemm_pipe_supported(a) || a.n <= 4096 || (a.type == kQ8_0 && a.x_f32 && a.m <= 16);
+  return gemm_skinny_supported(a) && (!gemm_pipe_supported(a) || a.n <= 4096);
 }
 
 template <int TYPE, typename OutT>
 static hipError_t launch_type(const GemvArgs& a, hipStream_t stream) {
   const GemmGroupArgs group = gemm_single(a);
   if (gemm_rows_takes(group, GemmPlan{0, 1})) return launch_gemm_rows(group, stream);
-  if (gemm_small_m(a)) return launch_gemm_skinny(a, stream);
+  if (gemm_skinny_supported(a)) return launch_gemm_skinny(a, stream);
   bool handled = false;
   const hipError_t status = launch_gemm_pipe(a, stream, &handled);
   if (handled) return status;

@@ -274,24 +274,19 @@ hipError_t launch_rows_type(GemmRowsLaunch& l, hipStream_t stream) {
 
 }  // namespace
 
+bool gemm_skinny_takes(const GemmGroupArgs& a) {
+  return a.m <= kSkinnyMaxM && a.count == 1 && gemm_skinny_better(a.type, a.m, a.n[0], a.k, a.x_f32);
+}
+
 // M <= 64, but
 //  * long rows with a K split across workgroups to take (a plan with a workspace) at M > 32, where every workgroup
 //    stages 16 or 32 whole activation rows for its few weight rows: 4096 x 12288 Q4_K at M = 64 31.4
 //    against 26.3 us, at M = 32 21.6 against 23.9;
-//  * one small matrix of the encodings that the per-element kernel (gemm_skinny) decodes cheaply, where
-//    latency is all: 1024 x 1024 at M = 16 Q8_0 4.8 against 4.2 us, Q2_K 4.7 against 4.0, but
-//    Q6_K 5.0 against 5.4, and 640 x 2560 Q8_0 7.6 against 8.2.
+//  * one matrix of short rows, where latency is all (gemm_skinny_better).
 bool gemm_rows_takes(const GemmGroupArgs& a, const GemmPlan& plan) {
   if (a.m > 64 || a.k > kRowsMaxK) return false;
   if (a.m > 32 && a.k >= 8192 && plan.small_m && plan.splits > 1) return false;
-  if (a.count > 1 || a.k > 1024) return true;
-  const int64_t elements = (int64_t)a.n[0] * a.k;
-  switch (a.type) {
-    case kQ8_0: return elements > (int64_t)4 << 20;
-    case kQ4_0: case kQ4_1: case kQ5_1: case kQ2_K: return elements >= (int64_t)4 << 20;
-    case kQ4_K: return a.m > 12 || elements >= (int64_t)4 << 20;
-    default: return true;
-  }
+  return !gemm_skinny_takes(a);
 }
 
 hipError_t launch_gemm_rows(const GemmGroupArgs& a, hipStream_t stream) {

@@ -170,7 +170,10 @@ bool gemm_rows_takes(const GemmGroupArgs& args, const GemmPlan& plan);
 hipError_t launch_gemm_rows(const GemmGroupArgs& args, hipStream_t stream);
 // One matrix as a group.
 GemmGroupArgs gemm_single(const GemvArgs& args);
-// Whether launch_gemm takes the small-M kernel for this shape.
+// Whether one matrix of this shape is left to the small-M kernel.
+bool gemm_skinny_takes(const GemmGroupArgs& args);
+// What tensor_gguf_gemm_plan_v1 counts as a matrix without a pipelined plan of its own: M <= 64, for shapes that the
+// pipelined tiles take also N <= 4096.
 bool gemm_small_m(const GemvArgs& args);
 
 }  // namespace tensor_gguf

@@ -69,6 +69,35 @@ inline GemmRowsPlan plan_gemm_rows(const int* n, int count, int m, int k, double
   return best;
 }
 
+// Whether one matrix is left to the per-element kernel (gemm_skinny): short rows, where latency is all and the streaming
+// kernel starts and ends ~1 us later.  It decodes per element, so the encodings differ in how long a row may be; K of
+// its 512-column passes counts against it, and for the streaming kernel whole rounds of 256-column steps over its waves (K = 512
+// and 1024 are, 544 to 768 and 1792 leave waves idle), hence the exceptions.  From graph replays of both
+// kernels, every encoding, M = 2 to 64, 320 to 20000 rows of 256 to 4096 columns, fp16 and fp32 x: the choice takes 0.1%
+// more than the better one on average (5% at the 99th percentile), with lines on elements 3.0%.  us, per element /
+// streaming, M = 16: Q2_K 8192 x 256 4.0 / 4.7, Q4_K 1024 x 1024 4.1 / 4.6 and 320 x 256 3.1 / 4.3, Q6_K 4096 x 512
+// 5.2 / 5.0; Q5_1 4096 x 1056 at M = 48 5.1 / 6.8, Q4_K 2560 x 2560 at M = 32 10.0 / 7.1.
+inline bool gemm_skinny_better(int type, int m, int n, int k, bool x_f32) {
+  // how the decode per element compares: cheap, Q4_K, Q5_0, dear
+  const int c = type == kQ4_K ? 1 : type == kQ5_0 ? 2 : type == kQ3_K || type == kQ5_K || type == kQ6_K ? 3 : 0;
+  const bool idle = (k + 255) / 256 == 7;
+  if (n <= 4096) {
+    if (m > 32 && n > 1024) {  // the streaming kernel spreads M over workgroups, each decoding again
+      constexpr int longest[4] = {1792, 1280, 1280, 768};
+      return k <= longest[c] && !(k == 1024 && (c >= 1 || x_f32));
+    }
+    if (c == 1 && m > 16 && n > 1024) return k < 512;
+    if (c == 2) return k <= 768 && k != 512;
+    return c == 0 ? k <= 1280 || (type == kQ5_1 && idle) : k <= (c == 1 ? 1024 : 511);
+  }
+  if (n <= 8192) {
+    if (m <= 16) return c <= 1 && (k <= 384 || (c == 0 && type != kQ4_0 && k % 256 != 0 && k <= 1056));
+    if (c == 0) return (k <= 1280 && k != 1024) || (idle && type != kQ4_0);
+    return k <= (c == 2 ? (m > 32 ? 544 : 768) : 512);
+  }
+  return c == 0 && m > 16 && m <= 32 && (long long)n * k <= 13ll << 19;
+}
+
 // The decode GEMV's workgroups: `groups` row tiles (or gate / up tile pairs) of one matrix and at most
 // `waves` waves.
 struct GemvRowsPlan {

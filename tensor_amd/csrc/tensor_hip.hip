@@ -604,14 +604,15 @@ int32_t gemm_group_call(const TensorCallV1* call, TensorErrorV1* error, bool has
   if (int32_t s = check_device(call, error)) return s;
   hipStream_t stream = reinterpret_cast<hipStream_t>(call->stream.handle);
   const bool rows = !forced && tensor_gguf::gemm_rows_takes(group, plan);
+  const bool skinny = !forced && !rows && tensor_gguf::gemm_skinny_takes(group);
   ScratchLease lease;
-  if (!has_workspace && !rows) {
+  if (!has_workspace && !rows && !skinny) {
     if (int32_t s = lease.acquire(call, stream, error)) return s;
     workspace = lease.address();
   }
   hipError_t status = hipSuccess;
   tensor_gguf::GemvArgs one[tensor_gguf::kGemmGroupMax];
-  bool small = true;  // every matrix on the small-M kernel, as tensor_gguf_gemm_v1 would run it
+  bool small = true;  // every matrix on the small-M kernel where no plan asks for another
   for (int i = 0; i < count; ++i) {
     one[i].x = group.x;
     one[i].w = group.w[i];
@@ -625,17 +626,17 @@ int32_t gemm_group_call(const TensorCallV1* call, TensorErrorV1* error, bool has
   }
   if (rows) {
     status = tensor_gguf::launch_gemm_rows(group, stream);
-  } else if ((!small || plan.small_m) && tensor_gguf::gemm_group_pipelined(group, plan)) {
+  } else if (!skinny && (!small || plan.small_m) && tensor_gguf::gemm_group_pipelined(group, plan)) {
     status = tensor_gguf::launch_gemm_group_plan(group, plan, workspace, workspace_bytes, stream);
-  } else if (!small && tensor_gguf::gemm_group_more(group)) {
+  } else if (!skinny && !small && tensor_gguf::gemm_group_more(group)) {
     status = tensor_gguf::launch_gemm_group_more(group, stream);
   } else {
-    // the other encodings and shapes, and small M where the plan keeps the small-M kernel, one
-    // launch per matrix in order (no workspace: such plans never split K)
+    // the other encodings and shapes, and one matrix on the small-M kernel, one launch per matrix in
+    // order (no workspace: such plans never split K)
     for (int i = 0; i < count && status == hipSuccess; ++i) status = tensor_gguf::launch_gemm(one[i], stream);
   }
   if (status != hipSuccess) return hip_fail(error, status, "GGUF grouped GEMM launch");
-  return has_workspace || rows ? TENSOR_OK : lease.release(stream, error);
+  return has_workspace || rows || skinny ? TENSOR_OK : lease.release(stream, error);
 }
 
 }  // namespace

@@ -707,22 +707,40 @@ def test_gemm_one_hot_rows_on_the_256_row_tiles(hip_device, c_oracle, encoding, 
     ("q4_0", 9, 5, 96, "float16"),         # N < 16: every row index clamped, a half chunk
 ])
 def test_gemm_small_m_kernel(hip_device, c_oracle, encoding, m, n, k, x_dtype):
-    """M <= 64 (every encoding; the pipelined tiles keep N > 4096): weights decoded
-    into MFMA operands, K over the waves of a workgroup, activations through a wave-private LDS
-    tile.  Every output row against the prefill oracle (fp16 x and W, fp32 sums)."""
+    """M <= 64, every encoding, on the small-M kernel (short rows: weights decoded into MFMA operands, K over
+    the waves of a workgroup, activations through a wave-private LDS tile) or the streaming kernel.
+    Every output row against the prefill oracle (fp16 x and W, fp32 sums)."""
     note("gemm-small-m", encoding, m, n, k, x_dtype)
     check_packed_rows(hip_device, c_oracle, encoding, m, n, k, x_dtype, 600 + m)
 
 
 @pytest.mark.parametrize("encoding,m,n,k,x_dtype", [
-    ("q4_0", 32, 8192, 2048, "float16"),   # N > 4096: the pipelined tiles
-    ("q8_0", 48, 6000, 1024, "float32"),   # pipelined, ragged M and N, fp32 x rounded as staged
-    ("q8_0", 16, 6000, 1024, "float32"),   # Q8_0 with fp32 x at M <= 16: the small-M kernel
-    ("q4_0", 20, 5000, 1056, "float16"),   # K % 64 == 32: the small-M kernel at any N
+    ("q8_0", 33, 8192, 1056, "float32"),   # three M tiles, two 16-row tiles of W per workgroup, K % 64 == 32
+    ("q4_1", 24, 12288, 512, "float16"),   # the widest N
+    ("q2_k", 40, 7000, 768, "float32"),
+    ("q4_k", 64, 1000, 1024, "float16"),   # four M tiles, one per workgroup
+    ("q4_k", 48, 4096, 1280, "float16"),   # all M tiles in each workgroup
+    ("q5_1", 64, 4096, 1792, "float16"),   # the longest rows
+    ("q6_k", 64, 4000, 768, "float32"),
+    ("q5_k", 16, 3000, 256, "float16"),
+    ("q3_k", 7, 2000, 256, "float16"),
+    ("q5_0", 20, 500, 544, "float32"),
+])
+def test_gemm_small_m_kernel_at_the_sizes_it_keeps(hip_device, c_oracle, encoding, m, n, k, x_dtype):
+    """One matrix of short rows, which the streaming kernel leaves to the small-M kernel."""
+    note("gemm-small-m-kept", encoding, m, n, k, x_dtype)
+    check_packed_rows(hip_device, c_oracle, encoding, m, n, k, x_dtype, 620 + m)
+
+
+@pytest.mark.parametrize("encoding,m,n,k,x_dtype", [
+    ("q4_0", 32, 8192, 2048, "float16"),   # the streaming kernel
+    ("q8_0", 48, 6000, 1024, "float32"),   # streaming, ragged M and N, fp32 x rounded as staged
+    ("q8_0", 16, 6000, 1024, "float32"),
+    ("q4_0", 20, 5000, 1056, "float16"),   # K % 64 == 32, M > 16: the small-M kernel
 ])
 def test_gemm_small_m_at_wide_n(hip_device, c_oracle, encoding, m, n, k, x_dtype):
     """M <= 64 with N > 4096, on either side of the boundary between the small-M kernel and the
-    pipelined tiles: every output row against the prefill oracle."""
+    streaming kernel: every output row against the prefill oracle."""
     note("gemm-small-m-wide", encoding, m, n, k, x_dtype)
     check_packed_rows(hip_device, c_oracle, encoding, m, n, k, x_dtype, 650 + m)
 
@@ -1012,17 +1030,18 @@ def run_gemm_group(device, encoding, x, raws, out_dtype, workspace_bytes=None):
     ("q4_k", 256, 4096, (4096,), False),             # o: 64 x 64 tiles with the K range inside the workgroup
     ("q5_k", 300, 8192, (1000, 77), True),           # ragged M and N, Q5_K
     ("q6_k", 200, 8192, (300, 500, 64), True),       # three ragged matrices, K >= 8192
-    ("q8_0", 64, 1024, (300, 100), False),           # small M: one small-M launch per matrix
+    ("q8_0", 64, 1024, (300, 100), False),           # small M: the streaming kernel, here and below up to M = 64
     ("q8_0", 256, 12288, (4096,), True),             # Q8_0 down at M=256: K split across workgroups
     ("q4_0", 256, 4096, (4096, 1024, 1024), True),   # Q4_0 q + k + v in one split launch
     ("q4_0", 200, 1056, (300, 500), False),          # K % 64 == 32: one generic launch per matrix
-    ("q4_k", 32, 4096, (4096, 1024, 1024), True),    # q + k + v at M=32: 64 x 64 tiles, K split 2 ways
+    ("q4_k", 32, 4096, (4096, 1024, 1024), True),    # q + k + v at M=32: streaming, the split plan unused
     ("q6_k", 48, 12288, (4096,), True),              # down at M=48: 64 x 64 tiles, K split 4 ways
     ("q4_0", 16, 4096, (4096, 1024, 1024), True),    # Q4_0 q + k + v at M=16
-    ("q6_k", 48, 2048, (3000, 100), False),          # small M, 98 workgroups at most: small-M kernel per matrix
-    ("q4_k", 32, 1024, (1024,), False),              # the showcase's shape: small-M kernel
+    ("q6_k", 48, 2048, (3000, 100), False),
+    ("q4_k", 32, 1024, (1024,), False),              # one matrix of the showcase's shape: small-M kernel
+    ("q2_k", 24, 256, (8192,), False),               # the same at N > 4096
     ("q8_0", 100, 12288, (4096,), True),             # down at M=100: 256 x 128 tiles, K split 8 ways
-    ("q4_k", 32, 4096, (12288, 12288), False),       # gate + up at M=32: 64 x 64 tiles, K over 2 wave groups
+    ("q4_k", 32, 4096, (12288, 12288), False),       # gate + up at M=32: streaming
     ("q4_k", 128, 4096, (12288, 12288), False),      # gate + up at M=128: 128 x 128 tiles, K over 2
     ("q4_k", 160, 4096, (4096, 1024, 1024), True),   # q + k + v at M=160: K split 4 ways
 ])

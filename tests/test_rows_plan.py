@@ -25,6 +25,7 @@ extern "C" void gemv_rows(const int* n, int count, int m, int pair, int* out) {
 extern "C" int gemv_group(const int* n, int count, int m, int k) { return gemv_rows_group_better(n, count, m, k); }
 extern "C" int gemv_single(int type, int m, int n, int k) { return gemv_rows_single_better(type, m, n, k); }
 extern "C" int gemv_pair(int type, int m, int n, int k) { return gemv_rows_pair_better(type, m, n, k); }
+extern "C" int gemm_skinny(int type, int m, int n, int k, int f32) { return gemm_skinny_better(type, m, n, k, f32); }
 """
 
 
@@ -143,3 +144,23 @@ def test_swiglu_pairs_of_one_pass_rows_stay_on_the_vector_kernels(library):
                                     ("q4_0", 1, 6912, 2560, True), ("q4_k", 2, 1, 256, True),
                                     ("q5_k", 1, 4096, 4096, False)):
         assert bool(library.gemv_pair(Q.ggml_type(encoding), m, n, k)) == rows, (encoding, m, n, k)
+
+
+@pytest.mark.parametrize("encoding,m,n,k,skinny", [
+    ("q2_k", 32, 8192, 256, True), ("q5_1", 12, 8192, 256, True), ("q5_1", 48, 4096, 1056, True),
+    ("q8_0", 64, 3000, 1056, True), ("q4_k", 16, 1024, 1024, True), ("q4_k", 64, 320, 256, True),
+    ("q6_k", 16, 640, 256, True), ("q5_0", 48, 2560, 1056, True), ("q4_1", 24, 12288, 512, True),
+    ("q6_k", 16, 4096, 512, False), ("q4_k", 32, 2560, 2560, False), ("q3_k", 9, 1024, 512, False),
+    ("q8_0", 16, 8192, 512, False), ("q2_k", 16, 20000, 256, False), ("q5_0", 32, 8192, 1056, False),
+])
+def test_streaming_gemm_leaves_short_rows_to_the_small_m_kernel(library, encoding, m, n, k, skinny):
+    """Both kernels timed at each."""
+    assert bool(library.gemm_skinny(Q.ggml_type(encoding), m, n, k, 0)) == skinny
+
+
+def test_small_m_kernel_keeps_no_long_rows(library):
+    for encoding in ("q4_0", "q5_0", "q4_k", "q3_k"):
+        for m in (2, 9, 32, 64):
+            for n in (1, 1024, 4096, 8192, 151936):
+                assert not library.gemm_skinny(Q.ggml_type(encoding), m, n, 2048, 0)
+                assert not library.gemm_skinny(Q.ggml_type(encoding), m, 151936, 256, 1)
