@@ -44,6 +44,17 @@ def check(got, x, w, what):
     assert (np.abs(got - xd @ wd.T) <= bound).all(), what
 
 
+def check_sums(got, x, w, what):
+    """Relative L2 against fp64: a sum rounds a few dozen times by at most 2^-24 of a partial sum, errors of
+    independent signs (random terms), so 2^-20 leaves a factor of ten.  The last step of 256 columns is far more of the
+    sums than that: a kernel that left it out would miss."""
+    xd, wd = x.astype(np.float16).astype(np.float64), w.astype(np.float64)
+    last, want = (x.shape[1] - 1) // 256 * 256, xd @ wd.T
+    bound = 2.0 ** -20 * np.linalg.norm(want)
+    assert np.linalg.norm(xd[:, last:] @ wd[:, last:].T) > 1000 * bound, what
+    assert np.linalg.norm(got - want) <= bound, what
+
+
 @pytest.mark.parametrize("encoding", ENCODINGS)
 def test_one_hot_rows_give_the_fp16_weights(hip_device, encoding):
     lengths = (32, 96, 1056) if Q.GEOMETRY[Q.ggml_type(encoding)][0] == 32 else (256, 768)
@@ -85,6 +96,24 @@ def test_launch_shapes(hip_device, encoding, m, rows, k):
     x = cases.activation(m, k, 82)
     for got, raw, n in zip(group(hip_device, encoding, x, raws), raws, rows):
         check(got, x, weights(encoding, raw, n, k), (encoding, m, n, k))
+        check_sums(got, x, weights(encoding, raw, n, k), (encoding, m, n, k))
+
+
+@pytest.mark.parametrize("encoding,m,k", [("q8_0", 32, 16416), ("q5_1", 64, 8224), ("q6_k", 40, 9472)])
+def test_every_step_of_long_rows_is_multiplied_once(hip_device, encoding, m, k):
+    """One-hot activations at the first and last column of every step of 256, so on both sides of every slice
+    boundary and in the short last step: each output is one fp16 weight, exactly."""
+    print("[gemm-rows] long rows, one-hot", encoding, m, k, flush=True)
+    rows = (48, 16)
+    raws = [cases.random_blocks(encoding, n, k, 85 + i) for i, n in enumerate(rows)]
+    steps = range(0, k, 256)
+    columns = sorted({*steps, *(min(s + 255, k - 1) for s in steps)})
+    for first in range(0, len(columns), m):
+        at = [columns[min(first + i, len(columns) - 1)] for i in range(m)]
+        x = np.zeros((m, k), np.float16)
+        x[np.arange(m), at] = 1.0
+        for got, raw, n in zip(group(hip_device, encoding, x, raws), raws, rows):
+            assert np.array_equal(got, weights(encoding, raw, n, k).astype(np.float32)[:, at].T), (n, at)
 
 
 @pytest.mark.parametrize("encoding,m,n,k", [("q6_k", 2, 300, 768), ("q4_k", 33, 1030, 2560), ("q5_0", 64, 77, 1056)])

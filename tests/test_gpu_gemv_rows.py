@@ -46,6 +46,15 @@ def reference(x, raw, encoding, n, k):
     return x @ w.T, k * 2.0 ** -24 * 3 * np.abs(x).sum(1)[:, None] * np.abs(w).max(1)[None, :] + 1e-12
 
 
+def check_sums(got, want, tail, what):
+    """Relative L2 against fp64 of sums over random terms: each rounds a few dozen times by at most 2^-24 of a
+    partial sum, errors of independent signs, so 2^-20 leaves a factor of ten.  tail, the part of the sums that the last
+    step adds, is far more than that: a kernel that left it out would miss."""
+    bound = 2.0 ** -20 * np.linalg.norm(want)
+    assert np.linalg.norm(tail) > 1000 * bound, what
+    assert np.linalg.norm(got - want) <= bound, what
+
+
 def check(got, x, raw, encoding, n, k, what):
     want, bound = reference(x, raw, encoding, n, k)
     assert not np.isnan(got).any(), what
@@ -88,8 +97,33 @@ def test_launch_shapes(hip_device, encoding, m, rows, k):
     note("shape", encoding, m, rows, k)
     raws = [cases.weight(n, k, encoding, 31 + i) for i, n in enumerate(rows)]
     x = cases.activation(m, k, 33)
+    last = (k - 1) // 256 * 256  # the last step's first column
     for got, raw, n in zip(run(hip_device, "gguf_gemv_group", x, raws, encoding, rows, count=2), raws, rows):
         check(got, x, raw, encoding, n, k, (encoding, m, n, k))
+        w = R.dequantize(raw, Q.ggml_type(encoding), n, k).astype(np.float64)
+        xd = x.astype(np.float64)
+        check_sums(got, xd @ w.T, xd[:, last:] @ w[:, last:].T, (encoding, m, n, k))
+
+
+@pytest.mark.parametrize("encoding,m,rows,k", [("q8_0", 8, (33, 16), 16416), ("q2_k", 7, (48, 5), 24832),
+                                               ("q5_1", 5, (17, 1), 30752), ("q4_k", 6, (20, 3), 26880)])
+def test_every_step_of_long_rows_is_multiplied_once(hip_device, encoding, m, rows, k):
+    """Rows whose activations are staged in slices: one-hot activations at the first and last column of every step of
+    256, so on both sides of every slice boundary and in the short last step.  An output is one weight, scale * code +
+    low: at most eight roundings of terms that are together at most 3 max |w|."""
+    note("long rows, one-hot", encoding, m, rows, k)
+    raws = [cases.weight(n, k, encoding, 35 + i) for i, n in enumerate(rows)]
+    ws = [R.dequantize(raw, Q.ggml_type(encoding), n, k).astype(np.float64) for raw, n in zip(raws, rows)]
+    steps = range(0, k, 256)
+    columns = sorted({*steps, *(min(s + 255, k - 1) for s in steps)})
+    for first in range(0, len(columns), m):
+        at = [columns[min(first + i, len(columns) - 1)] for i in range(m)]
+        x = np.zeros((m, k), np.float16)
+        x[np.arange(m), at] = 1.0
+        for got, w in zip(run(hip_device, "gguf_gemv_group", x, raws, encoding, rows, count=2), ws):
+            want, bound = w[:, at].T, 8 * 2.0 ** -24 * 3 * np.abs(w).max(1)[None, :]
+            assert not np.isnan(got).any() and (np.abs(got - want) <= bound).all(), at
+            assert (np.abs(want) > 1000 * bound).mean() > 0.5  # a step left out would be seen
 
 
 @pytest.mark.parametrize("encoding,m,n,k", [("q4_0", 5, 4100, 1056), ("q8_0", 8, 4100, 1056), ("q3_k", 3, 1300, 2816),
@@ -120,16 +154,17 @@ def test_swiglu_pairs(hip_device, encoding, m, n, k):
 
 @pytest.mark.parametrize("encoding", ENCODINGS)
 def test_sums_keep_fp32_precision(hip_device, encoding):
-    """Against fp64 over all outputs: each rounds a few dozen times by at most 2^-24 of a partial sum,
-    errors of independent signs (random activations), so 2^-20 relative L2 leaves a factor of ten; sums in
-    the precision of 16-bit exponent-aligned products would miss it by another ten."""
+    """Against fp64 over all outputs: sums in the precision of 16-bit exponent-aligned products would miss the
+    bound of check_sums by another ten, as they would at activations that are all fp16 subnormals (2^-16 times normal ones)
+    if those lost bits to their leading zeros."""
     m, rows, k = 3, (512, 512), 2560
     note("precision", encoding, m, rows, k)
     raws = [cases.weight(n, k, encoding, 77 + i) for i, n in enumerate(rows)]
-    x = np.random.default_rng(78).standard_normal((m, k)).astype(np.float16)
-    for got, raw, n in zip(run(hip_device, "gguf_gemv_group", x, raws, encoding, rows, count=2), raws, rows):
-        want, _ = reference(x, raw, encoding, n, k)
-        assert np.linalg.norm(got - want) <= 2.0 ** -20 * np.linalg.norm(want), encoding
+    for scale in (1.0, 2.0 ** -16):
+        x = (scale * np.random.default_rng(78).standard_normal((m, k))).astype(np.float16)
+        for got, raw, n in zip(run(hip_device, "gguf_gemv_group", x, raws, encoding, rows, count=2), raws, rows):
+            want, _ = reference(x, raw, encoding, n, k)
+            check_sums(got, want, want, (encoding, scale))
 
 
 def by_elements(x, w):

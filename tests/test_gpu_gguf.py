@@ -606,7 +606,7 @@ def test_c5_layer_chained_in_one_graph(hip_device, c_oracle, m):
     (520, 4096, 512),    # 128x128, K split 2, ragged M
     (384, 7168, 768),    # 128x128 unsplit (12 K steps do not split evenly)
     (256, 9984, 768),    # 128x64 unsplit
-    (80, 1000, 768),     # 64x64 unsplit, ragged N (M <= 64 at N <= 4096 takes the small-M kernel)
+    (80, 1000, 768),     # 64x64 unsplit, ragged N
     (80, 1000, 512),     # 64x64, K split 2
     (256, 9984, 1024),   # 64x64, K split 4
     (300, 11000, 512),   # 256x96 (one round of 230 workgroups against 172 of 256x128), ragged M and N
@@ -627,12 +627,12 @@ def test_gemm_tile_configurations(hip_device, c_oracle, encoding, m, n, k):
 
 @pytest.mark.parametrize("encoding,m,n,k", [
     ("q4_k", 96, 12288, 4096),    # 128 x 64 tiles, K over 2 wave groups (M <= 128)
-    ("q6_k", 40, 20480, 1024),    # 64 x 64 tiles, K over 2 (M <= 64 and >= 256 tiles)
+    ("q6_k", 40, 20480, 1024),    # the streaming kernel (M <= 64)
     ("q8_0", 100, 70000, 512),    # 128 x 128 unsplit (>= 512 tiles at M <= 128), ragged M and N
     ("q4_0", 130, 20480, 2048),   # 256 x 128 again from M = 129 (160 tiles)
 ])
 def test_gemm_tiles_at_small_m(hip_device, c_oracle, encoding, m, n, k):
-    """Tiles no more than twice as tall as M: shapes that select each of them below M = 129."""
+    """Tiles no more than twice as tall as M, from M = 65; the streaming kernel below."""
     code = Q.ggml_type(encoding)
     note("gemm-small-m-tiles", encoding, m, n, k)
     raw = cases.weight(n, k, encoding, 95)
@@ -694,8 +694,8 @@ def test_gemm_one_hot_rows_on_the_256_row_tiles(hip_device, c_oracle, encoding, 
 
 @pytest.mark.parametrize("encoding,m,n,k,x_dtype", [
     ("q4_0", 2, 1000, 1056, "float32"),    # ragged N, a last half chunk of K (K % 64 == 32)
-    ("q8_0", 33, 8200, 1056, "float32"),   # three M tiles, two 16-row tiles per workgroup
-    ("q4_k", 64, 4096, 2048, "float16"),   # four M tiles, the widest N of the K-quants
+    ("q8_0", 33, 8200, 1056, "float32"),   # three M tiles, ragged N
+    ("q4_k", 64, 4096, 2048, "float16"),   # four M tiles
     ("q6_k", 48, 1000, 4096, "float32"),
     ("q5_k", 16, 3000, 1024, "float16"),
     ("q2_k", 40, 9000, 768, "float32"),
@@ -836,11 +836,12 @@ def test_fp16_weights_are_the_cast_of_the_fp32_dequantization(hip_device, c_orac
 @pytest.mark.parametrize("encoding,k", [(e, 512) for e in MORE] + [
     ("q8_0", 544),    # 17 K steps: odd, so the pipelined kernel passes the shape on
     ("q4_0", 1056),   # K % 64 == 32
+    ("q4_1", 544), ("q5_0", 544), ("q5_1", 1056),
 ])
 def test_generic_gemm_one_hot_rows_give_dequantized_weights(hip_device, c_oracle, encoding, k):
-    """The generic GEMM stages every weight of the other encodings, and of Q8_0 / Q4_0 where K
-    is not an even number of 64-element steps, as fp16(dequant): one-hot rows read them back
-    bit for bit."""
+    """The generic GEMM stages every weight of the 32-element encodings where K is not an even number
+    of 64-element steps (at K = 512 the pipelined kernel does) as fp16(dequant): one-hot rows read
+    them back bit for bit."""
     code = Q.ggml_type(encoding)
     n = 384
     note("gemm-one-hot-generic", encoding, k)
@@ -853,11 +854,31 @@ def test_generic_gemm_one_hot_rows_give_dequantized_weights(hip_device, c_oracle
     assert np.array_equal(got, deq[:, perm].T), encoding
 
 
+@pytest.mark.parametrize("encoding", [e for e in MORE if e != "q5_k"])
+def test_generic_gemm_of_fp32_activations_gives_dequantized_weights(hip_device, c_oracle, encoding):
+    """The encodings without plans take the generic GEMM wherever x is fp32 (the packed form) and M > 64."""
+    code = Q.ggml_type(encoding)
+    n, k = 200, 512
+    note("gemm-one-hot-generic-fp32", encoding)
+    raw = cases.random_blocks(encoding, n, k, 101)
+    deq = c_oracle.dequantize(raw, code, n, k).astype(np.float16).astype(np.float32)
+    perm = np.random.default_rng(102).permutation(k)
+    x = np.zeros((k, k), np.float32)
+    x[np.arange(k), perm] = 1.0
+    exe = hip_device.load("gguf_packed", encoding=encoding, m=k, n=n, k=k)
+    xb, wb = hip_device.from_numpy(x.reshape(-1)), hip_device.from_numpy(raw.reshape(-1))
+    out = hip_device.empty((k * n,), "float32")
+    hip_device.fill_bytes(out, 0xFF)
+    exe.launch(xb, wb, out)
+    assert np.array_equal(out.to_numpy().reshape(k, n), deq[:, perm].T), encoding
+    for b in (xb, wb, out):
+        b.release()
+
+
 @pytest.mark.parametrize("m,n,k", [(4, 1003, 4096), (8, 12288, 4096), (2, 300, 8192), (3, 200, 2560)])
 def test_gemv_group_pair_of_equal_matrices(hip_device, m, n, k):
-    """Two Q4_K matrices of one shape at 2 <= M <= 4 (gate and up) in one grouped launch: the
-    multi-row kernel with a tile of each per workgroup (M = 8 and K = 2560 take one launch per
-    matrix)."""
+    """Two Q4_K matrices of one shape at 2 <= M <= 8 (gate and up) in one grouped launch of the
+    matrix-core decode kernel."""
     note("gemv-group-pair", m, n, k)
     x = cases.activation(m, k, 200 + m)
     raws = [cases.weight(n, k, "q4_k", 201 + i) for i in range(2)]
