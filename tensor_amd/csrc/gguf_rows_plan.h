@@ -73,8 +73,8 @@ inline GemmRowsPlan plan_gemm_rows(const int* n, int count, int m, int k, double
 // kernel starts and ends ~1 us later.  It decodes per element, so the encodings differ in how long a row may be; K of
 // its 512-column passes counts against it, and for the streaming kernel whole rounds of 256-column steps over its waves (K = 512
 // and 1024 are, 544 to 768 and 1792 leave waves idle), hence the exceptions.  From graph replays of both
-// kernels, every encoding, M = 2 to 64, 320 to 20000 rows of 256 to 4096 columns, fp16 and fp32 x: the choice takes 0.1%
-// more than the better one on average (5% at the 99th percentile), with lines on elements 3.0%.  us, per element /
+// kernels, every encoding, M = 2 to 64, 320 to 20000 rows of 256 to 4096 columns, fp16 and fp32 x: the choice takes 0.2%
+// more than the better one on average (6% at the 99th percentile), with lines on elements 3.0%.  us, per element /
 // streaming, M = 16: Q2_K 8192 x 256 4.0 / 4.7, Q4_K 1024 x 1024 4.1 / 4.6 and 320 x 256 3.1 / 4.3, Q6_K 4096 x 512
 // 5.2 / 5.0; Q5_1 4096 x 1056 at M = 48 5.1 / 6.8, Q4_K 2560 x 2560 at M = 32 10.0 / 7.1.
 inline bool gemm_skinny_better(int type, int m, int n, int k, bool x_f32) {
@@ -90,12 +90,17 @@ inline bool gemm_skinny_better(int type, int m, int n, int k, bool x_f32) {
     if (c == 2) return k <= 768 && k != 512;
     return c == 0 ? k <= 1280 || (type == kQ5_1 && idle) : k <= (c == 1 ? 1024 : 511);
   }
-  if (n <= 8192) {
-    if (m <= 16) return c <= 1 && (k <= 384 || (c == 0 && type != kQ4_0 && k % 256 != 0 && k <= 1056));
+  if (m <= 16) {
+    if (n > 8192) return c == 0 && k <= 256 && n <= 10240;
+    return c == 0 ? k <= 384 || (type != kQ4_0 && k % 256 != 0 && k <= 1056) : c <= 2 && k <= (c == 1 ? 384 : 256);
+  }
+  // beyond 4096 rows M's tiles stay in one workgroup, from 8192 with two tiles of W: one round of those only there
+  if (n < 8192) return m > 32 && k <= 256;
+  if (n == 8192) {
     if (c == 0) return (k <= 1280 && k != 1024) || (idle && type != kQ4_0);
     return k <= (c == 2 ? (m > 32 ? 544 : 768) : 512);
   }
-  return c == 0 && m > 16 && m <= 32 && (long long)n * k <= 13ll << 19;
+  return m <= 32 && (c == 0 ? (long long)n * k <= 13ll << 19 && k != 512 : c == 2 && k <= 256 && n <= 20480);
 }
 
 // The decode GEMV's workgroups: `groups` row tiles (or gate / up tile pairs) of one matrix and at most
@@ -126,8 +131,9 @@ inline GemvRowsPlan plan_gemv_rows(const int* n, int count, int m, bool pair) {
 // 6.2).  They lie where graph replays of both sides crossed, every encoding at 640 to 12288 rows of 512 to 6912 columns:
 // the choice costs up to 8% over the better one near a line, where lines on elements alone cost up to 34%.
 // A band of row lengths moves a line: up to 2048 columns are one pass of the Q4_0 and Q8_0 vector kernels, of which shorter
-// ones leave lanes idle (Q8_0 at M = 4: 3000 x 1536 4.1 us there, 4.5 here; 3000 x 2560 6.9 and 5.8), Q2_K's
-// gains at up to 1024, and Q6_K's from M = 3 beyond 2048 (1024 x 4096 at M = 3 5.0 there, 5.8 here).
+// ones leave lanes idle (Q8_0 at M = 4: 3000 x 1536 4.1 us there, 4.5 here; 3000 x 2560 6.9 and 5.8), at M = 2, 5 and 6
+// whole passes beyond too (Q4_0 5120 x 4096 at M = 2 5.5 and 6.3), and Q2_K's gain at up to 1024.  Q6_K's holds to one
+// round of waves of long rows, 2048 rows at M = 3 (x 4096 5.5 and 6.2, 2560 x 4096 6.9 and 5.9).
 inline bool gemv_rows_single_better(int type, int m, int n, int k) {
   const double millions = (double)n * k / (1 << 20), size2 = millions * millions * n / 4096;
   const int at = m <= 4 ? m - 1 : m <= 6 ? 4 : 5;
@@ -136,17 +142,20 @@ inline bool gemv_rows_single_better(int type, int m, int n, int k) {
   };
   const bool whole_step = m == 1 && k % 4096 == 0 && k <= 16384;  // row lengths of the tuned M = 1 kernels
   const bool half_step = m == 1 && k % 2048 == 0 && k <= 16384;
-  const double one_pass = k <= 1024 || k > 2048 ? 1 : m <= 2 ? 1.8 : 2.2;
+  const bool whole = (k > 1024 && k <= 2048) || (k % 2048 == 0 && (at == 1 || at == 4));
+  const double one_pass = !whole ? 1 : m <= 2 ? 1.8 : 2.2;
   switch (type) {
-    case kQ4_0: return !half_step && from({28, 16.5, 3.7, 2.5, 1, 0.5}, one_pass);
-    case kQ4_1: return !half_step && from({28, 24, 10, 6, 4, 2});
-    case kQ5_0: return !half_step && from({9, 5, 4, 2, 3.5, 0.75});
-    case kQ5_1: return !half_step && from({24, 10, 9, 6, 4, 3.5});
-    case kQ8_0: return !half_step && from({18, 18, 9, 3.5, 1.5, 0.75}, one_pass);
-    case kQ2_K: return !whole_step && from({18, 5, 5, 2, 3.5, 2}, k <= 1024 ? 2 : 1);
+    case kQ4_0: return !half_step && from({40, 16.5, 3.7, 2.5, 1, 0.5}, one_pass);
+    case kQ4_1: return !half_step && from({28, 21.5, 10, 6, 4, 2});
+    case kQ5_0: return !half_step && from({9, 4.9, 4, 2, 3.5, 0.75});
+    case kQ5_1: return !half_step && from({21.5, 10, 9, 6, 4, 3.5});
+    case kQ8_0: return !half_step && from({38.5, 18, 6, 3.5, 1.5, 0.75}, one_pass);
+    case kQ2_K: return !whole_step && from({18, 4.9, 4.9, 2, 3.5, 2}, k <= 1024 ? 2 : 1);
     case kQ3_K: return !whole_step && from({3.5, 2, 1.5, 1.5, 2, 1.5});
     case kQ5_K: return !whole_step && from({3, 2, 1.5, 0.75, 0.75, 0.75});
-    case kQ6_K: return !(whole_step && k <= 12288) && from({14, 0.5, 2.5, 0.5, 1.4, 0.5}, m >= 3 && k > 2048 ? 2.5 : 1);
+    case kQ6_K:
+      if (k > 2048 && (m == 3 ? n <= 2048 : at == 4 && n <= 1024)) return false;
+      return !(whole_step && k <= 12288) && from({13, 0.5, 2.5, 0.5, 1.2, 0.5});
     // M > 1: the plans of tensor_gguf_gemv_plan_v1.  M = 1: rows of 1024 columns are level, of 1536 and 2048 (one
     // pass there too) take 10 to 22% longer here, of 2560 to 6912 2 to 14% less.
     case kQ4_K: return m == 1 && !whole_step && k > 2048;

@@ -716,8 +716,8 @@ def test_gemm_small_m_kernel(hip_device, c_oracle, encoding, m, n, k, x_dtype):
 
 @pytest.mark.parametrize("encoding,m,n,k,x_dtype", [
     ("q8_0", 33, 8192, 1056, "float32"),   # three M tiles, two 16-row tiles of W per workgroup, K % 64 == 32
-    ("q4_1", 24, 12288, 512, "float16"),   # the widest N
-    ("q2_k", 40, 7000, 768, "float32"),
+    ("q4_1", 24, 12288, 384, "float16"),   # the widest N
+    ("q2_k", 40, 8192, 768, "float32"),
     ("q4_k", 64, 1000, 1024, "float16"),   # four M tiles, one per workgroup
     ("q4_k", 48, 4096, 1280, "float16"),   # all M tiles in each workgroup
     ("q5_1", 64, 4096, 1792, "float16"),   # the longest rows
@@ -736,7 +736,8 @@ def test_gemm_small_m_kernel_at_the_sizes_it_keeps(hip_device, c_oracle, encodin
     ("q4_0", 32, 8192, 2048, "float16"),   # the streaming kernel
     ("q8_0", 48, 6000, 1024, "float32"),   # streaming, ragged M and N, fp32 x rounded as staged
     ("q8_0", 16, 6000, 1024, "float32"),
-    ("q4_0", 20, 5000, 1056, "float16"),   # K % 64 == 32, M > 16: the small-M kernel
+    ("q4_0", 20, 5000, 1056, "float16"),   # K % 64 == 32
+    ("q4_0", 50, 5000, 256, "float16"),    # the small-M kernel
 ])
 def test_gemm_small_m_at_wide_n(hip_device, c_oracle, encoding, m, n, k, x_dtype):
     """M <= 64 with N > 4096, on either side of the boundary between the small-M kernel and the
