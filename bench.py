@@ -35,6 +35,10 @@ Also reported:
   C3 LM head, C4 prefill GEMM, C5 decoder-layer chain at M = 1 and M = 256),
   the showcase's packed call at its own shapes, and the resident-dequantized
   torch.mm lower bound (benchmark.py:478-488) measured in a torch-first child.
+
+The printed line holds the medians and rates of these, so that it stays under 8 KB and whole
+in a log's tail; everything else is logged on stderr as it is measured and written to the
+file that ``--full FILE`` names.
 """
 
 from __future__ import annotations
@@ -945,6 +949,29 @@ def gemv_plan_sweep(device, only=None):
     return report
 
 
+# -------------------------------------------------------------------- line --
+
+def printed(result):
+    """The record as printed: each case's median (or its per-call medians) and rates, without samples, extremes and
+    constants."""
+    rates = ("GB/s", "TFLOP/s", "GFLOP/s")
+
+    def brief(case):
+        if not isinstance(case, dict):
+            return case
+        kept = {k: v for k, v in case.items() if k in ("median_us", "per_group_us", "error", *rates)}
+        return kept or {k: brief(v) for k, v in case.items() if isinstance(v, dict)}
+
+    line = json.loads(json.dumps(result))
+    line["config"].get("step_us", {}).pop("samples_us", None)
+    line["details"] = {k: brief(v) for k, v in line["details"].items() if k != "measurement_order"}
+    if line["cpu_baseline"]:
+        line["cpu_baseline"]["per_config"] = {
+            name: {k: case[k] for k in ("ms", "single_thread_ms") if k in case}
+            for name, case in line["cpu_baseline"]["per_config"].items()}
+    return json.dumps(line, separators=(",", ":"))
+
+
 # ------------------------------------------------------------------- main --
 
 def main():
@@ -953,6 +980,7 @@ def main():
     parser.add_argument("--gpus", type=int, default=1)
     parser.add_argument("--steps", type=int, default=300)
     parser.add_argument("--warmup", type=int, default=20)
+    parser.add_argument("--full", metavar="FILE", help="also write the whole record, every sample in it, as JSON")
     parser.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline")
     parser.add_argument("--no-details", action="store_true", help="headline only")
     parser.add_argument("--no-torch", action="store_true", help="skip the resident-dequantized torch.mm leg")
@@ -1106,7 +1134,10 @@ def main():
         "cpu_baseline": None if args.no_cpu else cpu_baseline(args.cpu_seconds),
         "details": details,
     }
-    print(json.dumps(result))
+    if args.full:
+        with open(args.full, "w") as file:
+            json.dump(result, file, indent=1)
+    print(printed(result))
     return 0
 
 
