@@ -133,7 +133,8 @@ int32_t tensor_gguf_gemv_group_v1(const TensorCallV1 *call, TensorErrorV1 *error
  * workspace and a second kernel adds them in split order (deterministic) and converts; the
  * split is chosen to fit the workspace given (any size; a short one only limits the split).
  * Up to M = 64 the group runs on the streaming kernel in one launch, without that split, but for
- * rows of 8192 columns or more at M > 32 where a plan splits K.  Beyond it Q4_K, Q5_K, Q6_K, Q8_0 and
+ * rows of 8192 columns or more at M > 32 where a plan splits K; one matrix of short rows runs
+ * on the small-M kernel of tensor_gguf_gemm_v1.  Beyond it Q4_K, Q5_K, Q6_K, Q8_0 and
  * Q4_0 use the pipelined kernel (Q8_0 / Q4_0 where K is an even number of 64-element steps); Q4_1,
  * Q5_0, Q5_1, Q2_K and Q3_K use it without the split (no workspace); the other shapes
  * take one launch per matrix as tensor_gguf_gemm_v1 runs it.  Arguments, in order:
@@ -168,7 +169,7 @@ int32_t tensor_gguf_gemm_group_noalloc_v1(const TensorCallV1 *call, TensorErrorV
 /*
  * Workspace bytes the pipelined plan of tensor_gguf_gemm_group_v1 uses for this shape (0: it does
  * not split K): n[0 .. count-1] are the matrices' row counts.  Calls of M <= 64 that the streaming
- * kernel takes leave the workspace alone.
+ * or small-M kernel takes leave the workspace alone.
  */
 int32_t tensor_gguf_gemm_workspace_v1(uint32_t type, int64_t m, int64_t k, const int64_t *n, uint32_t count,
                                       uint64_t *bytes, TensorErrorV1 *error);
@@ -176,8 +177,8 @@ int32_t tensor_gguf_gemm_workspace_v1(uint32_t type, int64_t m, int64_t k, const
 /*
  * The pipelined plan of tensor_gguf_gemm_group_v1 for this shape given workspace_bytes of
  * workspace: the tile index and K split across workgroups, and whether there is one (0: each
- * matrix takes another kernel).  Up to M = 64 the streaming kernel replaces it but for rows of 8192
- * columns or more at M > 32 with a split; tensor_gguf_gemm_group_plan_v1 runs it at any M.  No counterpart in the
+ * matrix takes another kernel).  Up to M = 64 the streaming kernel (one matrix of short rows: the
+ * small-M kernel) replaces it but for rows of 8192 columns or more at M > 32 with a split; tensor_gguf_gemm_group_plan_v1 runs it at any M.  No counterpart in the
  * reference, whose showcase searches schedules per case (benchmarks/kernels/showcase/
  * benchmark.py:214-237): with the two entries below a caller re-times the plans the library
  * could take and checks the one it picks.

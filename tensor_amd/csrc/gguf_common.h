@@ -158,6 +158,11 @@ __device__ __forceinline__ float wave_sum(float v) {
   return rows_total(v);
 }
 
+// Bit i (0..3) of v to bit 4 of byte i (the fifth bits of four codes).
+__device__ __forceinline__ uint32_t fifth_bits(uint32_t v) {
+  return (__umul24(v & 15u, 0x00204081u) & 0x01010101u) << 4;
+}
+
 // Q4_K: the (scale, min) 6-bit pairs of sub-blocks 2j and 2j+1 from the three
 // scale dwords s0 = bytes 0-3, s1 = bytes 4-7, s2 = bytes 8-11.
 // Sub-blocks 0-3: scale = byte[s] & 63, min = byte[s+4] & 63.

@@ -14,11 +14,6 @@ namespace pipe {
 constexpr int BK = 64, ROW = 80;  // halves per LDS row (16-byte aligned, padded)
 constexpr float kTwo24 = 16777216.0f, kTwo20 = 1048576.0f;
 
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  const _Float16 ha = (_Float16)a, hb = (_Float16)b;
-  return (uint32_t)__builtin_bit_cast(uint16_t, ha) | ((uint32_t)__builtin_bit_cast(uint16_t, hb) << 16);
-}
-
 // fp16(scale * q + bias) for four codes q < 1024 given as fp16 subnormal pairs
 // p02 = (q0, q2) * 2^-24 and p13 = (q1, q3) * 2^-24 (a code masked into the low
 // bits of a half is that subnormal exactly). With scale24 = scale * 2^24 each
@@ -88,11 +83,6 @@ struct Geometry<kQ3_K, TPR> {
   static constexpr int QB = 32 / TPR;
   static constexpr int W0 = QB / 4, W1 = 3 + QB / 4;  // quants; scale bytes (two dwords), d, third bits
 };
-
-// Bit i (0..3) of v to bit 4 of byte i.
-__device__ __forceinline__ uint32_t spread_fifth(uint32_t v) {
-  return (__umul24(v & 15u, 0x00204081u) & 0x01010101u) << 4;
-}
 
 // fp16(scale * (q - OFFSET)) for the four byte codes of q: the offset comes off the subnormal codes
 // exactly (v_pk_add_f16), so an infinite scale stays infinite as in scale * (q - OFFSET).
@@ -337,8 +327,8 @@ __global__ __launch_bounds__(WM * WN * 64 * KS) void gemm_pipe(const XT* __restr
             uint32_t lo = ra[i] & 0x0F0F0F0Fu, hi = (ra[i] >> 4) & 0x0F0F0F0Fu;
             if constexpr (TYPE != kQ4_1) {
               const uint32_t fifth = rb[1] >> (j0 + 4 * i);
-              lo |= spread_fifth(fifth);
-              hi |= spread_fifth(fifth >> 16);
+              lo |= fifth_bits(fifth);
+              hi |= fifth_bits(fifth >> 16);
             }
             *reinterpret_cast<uint2*>(dst + 4 * i) = scaled4<OFFSET>(lo, d24, m);
             *reinterpret_cast<uint2*>(dst + 16 + 4 * i) = scaled4<OFFSET>(hi, d24, m);
@@ -521,9 +511,9 @@ __global__ __launch_bounds__(WM * WN * 64 * KS) void gemm_pipe(const XT* __restr
       // the x DMA of the fetched step is issued ahead of its weight loads and the order is pinned:
       // loads complete in order, so once a wave's dequant has waited on those weights (the next
       // step's store), its DMA'd x has landed too, before the barrier that follows.
-      // Ping-pong: the upper half of the waves (one weight part each) issue their MFMAs before
-      // they dequantize, the lower half (two parts) after, so the two waves that share a SIMD
-      // keep its matrix pipe and its VALU busy at the same time.
+      // Ping-pong: the upper half of the waves issue their MFMAs before they dequantize, the lower
+      // half (in the 256 x 192 tile those with two weight parts, everywhere else each wave has one) after, so
+      // the two waves that share a SIMD keep its matrix pipe and its VALU busy at the same time.
       auto mfma_all = [&]() {
         multiply(a1, b1);
         __builtin_amdgcn_sched_barrier(0);

@@ -2,8 +2,8 @@
 // fp16 activations: out[m, n] = sum_k x[m, k] * W[n, k], up to three matrices that share x in
 // one launch, or a gate / up pair with the SwiGLU epilogue.
 //
-// Each lane owns whole pieces of one weight row (a unit of 64 or 128 elements: two 32-element
-// blocks, or a quarter or half super-block), so that a piece's scale is a value of the lane's
+// Each lane owns whole pieces of one weight row (a unit of 64 elements: two 32-element
+// blocks, or a quarter super-block), so that a piece's scale is a value of the lane's
 // own and is applied once per 16 or 32 elements in fp32.  v_mfma_f32_16x16x32_f16 does the
 // products all the same: its B operand takes 8 codes from every lane (lane n + 16 g: row n of a
 // 16-row tile, piece g of four that follow each other), and its A operand holds the activations

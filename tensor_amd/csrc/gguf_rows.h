@@ -33,11 +33,6 @@ __device__ __forceinline__ half8_t operand(uint32_t lo, uint32_t hi) {
   return __builtin_bit_cast(half8_t, make_uint4(v[0], v[1], v[2], v[3]));
 }
 
-// Bit i (0..3) of v to bit 4 of byte i.
-__device__ __forceinline__ uint32_t spread4(uint32_t v) {
-  return (__umul24(v & 15u, 0x00204081u) & 0x01010101u) << 4;
-}
-
 constexpr float kTwo9 = 512.0f;  // the codes' 2^-9 is taken out in the scales
 
 // What differs between encodings.  ELEMS: elements of a unit (two blocks, or a quarter super-block); SUB: elements that share a scale;
@@ -133,8 +128,8 @@ struct Unit {
       uint32_t lo = (q[w] >> shift) & 0x0F0F0F0Fu, hi = (q[w + 1] >> shift) & 0x0F0F0F0Fu;
       if constexpr (TYPE == kQ5_0 || TYPE == kQ5_1) {
         constexpr int bit = 8 * (T & 3);  // chunk T is elements 8 (T & 3) of the block
-        lo |= spread4(h[2 + b] >> bit);
-        hi |= spread4(h[2 + b] >> (bit + 4));
+        lo |= fifth_bits(h[2 + b] >> bit);
+        hi |= fifth_bits(h[2 + b] >> (bit + 4));
       }
       return operand<TYPE == kQ4_0 ? 8 : TYPE == kQ5_0 ? 16 : 0>(lo, hi);
     } else if constexpr (TYPE == kQ2_K) {

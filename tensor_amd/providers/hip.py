@@ -430,8 +430,9 @@ class Device(Session):
 
     # -------------------------------------------------------------- graphs --
     def gemm_workspace(self, encoding, m: int, k: int, rows) -> int:
-        """Bytes of workspace ``gguf_gemm_group`` uses for this shape (``rows`` = each matrix's
-        N); 0 when it does not split K.  A smaller workspace is accepted and limits the split."""
+        """Bytes of workspace the pipelined plan of ``gguf_gemm_group`` uses for this shape (``rows`` = each
+        matrix's N); 0 when it does not split K.  A smaller workspace is accepted and limits the split;
+        calls of M <= 64 on the streaming or small-M kernel leave it alone."""
         from tensor_amd.gguf.quant import ggml_type
 
         rows = [int(n) for n in rows]
@@ -454,9 +455,11 @@ class Device(Session):
         return {"kernel": kernel.value, "name": GEMV_KERNELS[kernel.value], "a": a.value, "b": b.value}
 
     def gemm_plan(self, encoding, m: int, k: int, rows, workspace_bytes: int | None = None) -> dict:
-        """The plan ``gguf_gemm_group`` takes for this shape (``workspace_bytes`` of workspace,
+        """The pipelined plan of ``gguf_gemm_group`` for this shape (``workspace_bytes`` of workspace,
         by default as much as it asks for): tile index, its geometry, the K split, and whether
-        the pipelined kernel runs (otherwise each matrix takes the small-M kernel)."""
+        there is one.  Up to M = 64 ``gguf_gemm_group`` runs the streaming kernel instead (one matrix of short rows:
+        the small-M kernel), but for rows of 8192 columns or more at M > 32 with a split;
+        ``gguf_gemm_group_plan`` runs the plan at any M."""
         from tensor_amd.gguf.quant import ggml_type
 
         rows = [int(n) for n in rows]
