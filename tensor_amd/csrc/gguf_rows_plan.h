@@ -83,11 +83,11 @@ inline bool gemm_skinny_better(int type, int m, int n, int k, bool x_f32) {
   const bool idle = (k + 255) / 256 == 7;
   if (n <= 4096) {
     if (m > 32 && n > 1024) {  // the streaming kernel spreads M over workgroups, each decoding again
-      constexpr int longest[4] = {1792, 1280, 1280, 768};
-      return k <= longest[c] && !(k == 1024 && (c >= 1 || x_f32));
+      constexpr int longest[4] = {1280, 768, 1056, 768};
+      return (k <= longest[c] && !(k == 1024 && (c >= 1 || x_f32))) || (idle && c == 0 && n >= 3072);
     }
     if (c == 1 && m > 16 && n > 1024) return k < 512;
-    if (c == 2) return k <= 768 && k != 512;
+    if (c == 2) return k <= 768 && k != 512 && (k < 512 || n <= 1024);
     return c == 0 ? k <= 1280 || (type == kQ5_1 && idle) : k <= (c == 1 ? 1024 : 511);
   }
   if (m <= 16) {
@@ -95,10 +95,10 @@ inline bool gemm_skinny_better(int type, int m, int n, int k, bool x_f32) {
     return c == 0 ? k <= 384 || (type != kQ4_0 && k % 256 != 0 && k <= 1056) : c <= 2 && k <= (c == 1 ? 384 : 256);
   }
   // beyond 4096 rows M's tiles stay in one workgroup, from 8192 with two tiles of W: one round of those only there
-  if (n < 8192) return m > 32 && k <= 256;
+  if (n < 8192) return m > 32 && k <= 256 && type != kQ5_K;
   if (n == 8192) {
-    if (c == 0) return (k <= 1280 && k != 1024) || (idle && type != kQ4_0);
-    return k <= (c == 2 ? (m > 32 ? 544 : 768) : 512);
+    if (c == 0) return (k <= 1056 && k != 1024) || ((idle || k == 1280) && type != kQ4_0 && type != kQ4_1);
+    return k <= (type == kQ5_K ? 256 : c == 2 && m <= 32 ? 768 : 512);
   }
   return m <= 32 && (c == 0 ? (long long)n * k <= 13ll << 19 && k != 512 : c == 2 && k <= 256 && n <= 20480);
 }
@@ -128,11 +128,12 @@ inline GemvRowsPlan plan_gemv_rows(const int* n, int count, int m, bool pair) {
 // where latency is all (1024 x 1024 at M = 1: Q4_0 3.0 against 2.3 us).  A line for M = 1, 2, 3, 4, 5 to 6 and
 // 7 to 8, in 2^20 elements times sqrt(n / 4096): few rows leave CUs without a tile, so of two matrices of one size the
 // longer rows gain less (Q4_1 at M = 6: 1024 x 6912 9.5 us against 7.1 on the vector kernel, 4096 x 2048 5.4 against
-// 6.2).  They lie where graph replays of both sides crossed, every encoding at 640 to 12288 rows of 512 to 6912 columns:
-// the choice costs up to 8% over the better one near a line, where lines on elements alone cost up to 34%.
+// 6.2).  They lie where graph replays of both sides crossed, every encoding at 640 to 12288 rows of 512 to 6912 columns,
+// weights in the caches and out of them: the choice takes 1.1% more than the better one on average and up to 14% near a
+// line, where lines on elements alone took 3.3% and up to 34%.
 // A band of row lengths moves a line: up to 2048 columns are one pass of the Q4_0 and Q8_0 vector kernels, of which shorter
-// ones leave lanes idle (Q8_0 at M = 4: 3000 x 1536 4.1 us there, 4.5 here; 3000 x 2560 6.9 and 5.8), at M = 2, 5 and 6
-// whole passes beyond too (Q4_0 5120 x 4096 at M = 2 5.5 and 6.3), and Q2_K's gain at up to 1024.  Q6_K's holds to one
+// ones leave lanes idle (Q8_0 at M = 4: 3000 x 1536 4.1 us there, 4.5 here; 3000 x 2560 6.9 and 5.8), from M = 2 to
+// 6 whole passes beyond too (Q4_0 5120 x 4096 at M = 2 5.5 and 6.3), and Q2_K's gain at up to 1024.  Q6_K's holds to one
 // round of waves of long rows, 2048 rows at M = 3 (x 4096 5.5 and 6.2, 2560 x 4096 6.9 and 5.9).
 inline bool gemv_rows_single_better(int type, int m, int n, int k) {
   const double millions = (double)n * k / (1 << 20), size2 = millions * millions * n / 4096;
@@ -142,20 +143,20 @@ inline bool gemv_rows_single_better(int type, int m, int n, int k) {
   };
   const bool whole_step = m == 1 && k % 4096 == 0 && k <= 16384;  // row lengths of the tuned M = 1 kernels
   const bool half_step = m == 1 && k % 2048 == 0 && k <= 16384;
-  const bool whole = (k > 1024 && k <= 2048) || (k % 2048 == 0 && (at == 1 || at == 4));
-  const double one_pass = !whole ? 1 : m <= 2 ? 1.8 : 2.2;
+  const bool whole = (k > 1024 && k <= 2048) || (k % 2048 == 0 && at >= 1 && at <= 4);
+  const double one_pass = !whole ? 1 : m <= 2 ? 1.4 : 2.2;
   switch (type) {
-    case kQ4_0: return !half_step && from({40, 16.5, 3.7, 2.5, 1, 0.5}, one_pass);
-    case kQ4_1: return !half_step && from({28, 21.5, 10, 6, 4, 2});
-    case kQ5_0: return !half_step && from({9, 4.9, 4, 2, 3.5, 0.75});
-    case kQ5_1: return !half_step && from({21.5, 10, 9, 6, 4, 3.5});
-    case kQ8_0: return !half_step && from({38.5, 18, 6, 3.5, 1.5, 0.75}, one_pass);
-    case kQ2_K: return !whole_step && from({18, 4.9, 4.9, 2, 3.5, 2}, k <= 1024 ? 2 : 1);
-    case kQ3_K: return !whole_step && from({3.5, 2, 1.5, 1.5, 2, 1.5});
-    case kQ5_K: return !whole_step && from({3, 2, 1.5, 0.75, 0.75, 0.75});
+    case kQ4_0: return !half_step && from({38, 18, 3.8, 2.5, 1, 0.5}, one_pass);
+    case kQ4_1: return !half_step && from({28, 13.8, 8, 4.4, 3.6, 1.7});
+    case kQ5_0: return !half_step && from({5.7, 4.4, 3.6, 1.6, 1.7, 0.75});
+    case kQ5_1: return !half_step && from({18, 9.8, 5.7, 3.6, 3.6, 1.7});
+    case kQ8_0: return !half_step && from({20.6, 16.8, 6.1, 2.7, 1.3, 0.7}, one_pass);
+    case kQ2_K: return !whole_step && from({18, 4.7, 4.7, 1.6, 3.5, 0.75}, k > 1024 ? 1 : m == 2 && k > 512 ? 3 : 2);
+    case kQ3_K: return !whole_step && from({3.5, 1.6, 1.1, 1.1, 2, 0.75}, k <= 1024 ? 1.3 : 1);
+    case kQ5_K: return !whole_step && from({2, 1.6, 0.75, 0.55, 0.55, 0.55});
     case kQ6_K:
-      if (k > 2048 && (m == 3 ? n <= 2048 : at == 4 && n <= 1024)) return false;
-      return !(whole_step && k <= 12288) && from({13, 0.5, 2.5, 0.5, 1.2, 0.5});
+      if (k > 2048 && (m == 3 ? n <= 2048 && k <= 4096 : at == 4 && n <= 1024)) return false;
+      return !(whole_step && k <= 12288) && from({13, 0.5, 0.5, 0.5, 0.5, 0.5});
     // M > 1: the plans of tensor_gguf_gemv_plan_v1.  M = 1: rows of 1024 columns are level, of 1536 and 2048 (one
     // pass there too) take 10 to 22% longer here, of 2560 to 6912 2 to 14% less.
     case kQ4_K: return m == 1 && !whole_step && k > 2048;

@@ -719,7 +719,7 @@ def test_gemm_small_m_kernel(hip_device, c_oracle, encoding, m, n, k, x_dtype):
     ("q4_1", 24, 12288, 384, "float16"),   # the widest N
     ("q2_k", 40, 8192, 768, "float32"),
     ("q4_k", 64, 1000, 1024, "float16"),   # four M tiles, one per workgroup
-    ("q4_k", 48, 4096, 1280, "float16"),   # all M tiles in each workgroup
+    ("q4_k", 48, 4096, 768, "float16"),    # all M tiles in each workgroup
     ("q5_1", 64, 4096, 1792, "float16"),   # the longest rows
     ("q6_k", 64, 4000, 768, "float32"),
     ("q5_k", 16, 3000, 256, "float16"),
