@@ -81,12 +81,16 @@ inline bool gemm_skinny_better(int type, int m, int n, int k, bool x_f32) {
   // how the decode per element compares: cheap, Q4_K, Q5_0, dear
   const int c = type == kQ4_K ? 1 : type == kQ5_0 ? 2 : type == kQ3_K || type == kQ5_K || type == kQ6_K ? 3 : 0;
   const bool idle = (k + 255) / 256 == 7;
+  if (x_f32 && c == 0 && m > 16 && n > 1024 && k > 1056 && k <= 1536)  // 2560 x 1280 at M = 64: Q4_1 8.7 / 7.4 us,
+    return type == kQ2_K && m > 32;                                     // Q2_K 6.8 / 7.5
+  if (x_f32 && (type == kQ4_1 || type == kQ5_1) && m > 8 && m <= 32 && n <= 2048 && k > 1792 && k <= 2048)
+    return true;  // the lightest decode, and a streaming slice of fp32 x ends here: 2048 x 2048 7.4 / 8.3 us, Q5_1
   if (n <= 4096) {
     if (m > 32 && n > 1024) {  // the streaming kernel spreads M over workgroups, each decoding again
       constexpr int longest[4] = {1280, 768, 1056, 768};
       return (k <= longest[c] && !(k == 1024 && (c >= 1 || x_f32))) || (idle && c == 0 && n >= 3072);
     }
-    if (c == 1 && m > 16 && n > 1024) return k < 512;
+    if (c == 1 && n > 1024 && (m > 16 || x_f32)) return k < 512 || (m <= 16 && k == 512);
     if (c == 2) return k <= 768 && k != 512 && (k < 512 || n <= 1024);
     return c == 0 ? k <= 1280 || (type == kQ5_1 && idle) : k <= (c == 1 ? 1024 : 511);
   }

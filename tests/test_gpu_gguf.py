@@ -722,6 +722,7 @@ def test_gemm_small_m_kernel(hip_device, c_oracle, encoding, m, n, k, x_dtype):
     ("q4_k", 48, 4096, 768, "float16"),    # all M tiles in each workgroup
     ("q5_1", 64, 4096, 1792, "float16"),   # the longest rows
     ("q6_k", 64, 4000, 768, "float32"),
+    ("q5_1", 20, 2000, 2048, "float32"),
     ("q5_k", 16, 3000, 256, "float16"),
     ("q3_k", 7, 2000, 256, "float16"),
     ("q5_0", 20, 500, 544, "float32"),

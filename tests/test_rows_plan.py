@@ -160,6 +160,14 @@ def test_streaming_gemm_leaves_short_rows_to_the_small_m_kernel(library, encodin
     assert bool(library.gemm_skinny(Q.ggml_type(encoding), m, n, k, 0)) == skinny
 
 
+def test_fp32_activations_move_the_lines_of_the_small_m_kernel(library):
+    for encoding, m, n, k, half, single in (("q4_1", 32, 2560, 1280, 1, 0), ("q5_1", 32, 2048, 2048, 0, 1),
+                                            ("q8_0", 64, 4096, 1024, 1, 0), ("q4_0", 16, 2560, 1280, 1, 1)):
+        type_ = Q.ggml_type(encoding)
+        assert bool(library.gemm_skinny(type_, m, n, k, 0)) == bool(half), (encoding, m, n, k)
+        assert bool(library.gemm_skinny(type_, m, n, k, 1)) == bool(single), (encoding, m, n, k)
+
+
 def test_small_m_kernel_keeps_no_long_rows(library):
     for encoding in ("q4_0", "q5_0", "q4_k", "q3_k"):
         for m in (2, 9, 32, 64):
